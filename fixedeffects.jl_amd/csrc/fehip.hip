@@ -29,6 +29,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/fehip.h"
@@ -36,6 +37,7 @@
 #include "csr_build.h"
 #include "grouping.h"
 #include "fehip_common.h"
+#include "hostmem.h"
 #include "linmap.h"
 
 using namespace fehip;
@@ -133,7 +135,16 @@ struct fehip_solver {
     void *scale_all[2] = {nullptr, nullptr};  // p, every FE's scale, [0] double, [1] float
     int32_t *d_flag = nullptr;  // range-check flag
     int32_t *h_flag = nullptr;  // pinned
-    std::vector<void *> allocs;
+    // device blocks in use, with their size and device; and those given back
+    // on this handle: the stream's later work may use them again (it runs
+    // after what still reads them), other handles only once it is idle
+    // (release_spares)
+    struct Block {
+        size_t size;
+        int device;
+    };
+    std::unordered_map<void *, Block> allocs;
+    std::multimap<size_t, std::pair<void *, int>> spares;
     std::map<int, Plan *> plans;
     // sort scratch
     int32_t *sk[2] = {nullptr, nullptr}, *sv[2] = {nullptr, nullptr};
@@ -198,14 +209,24 @@ struct FwlScope {
 
 template <typename P>
 static int dalloc(fehip_solver *h, P **ptr, size_t count) {
+    const size_t bytes = std::max<size_t>(count, 1) * sizeof(P);
     void *q = nullptr;
-    hipError_t e = hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(P));
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return fail(FEHIP_EOOM, "hipMalloc of " + std::to_string(count * sizeof(P)) + " bytes failed: " +
-                                    hipGetErrorString(e));
+    fehip_solver::Block b{};
+    // a spare of up to a quarter more than asked for
+    auto it = h->spares.lower_bound(bytes);
+    if (it != h->spares.end() && it->first <= bytes + bytes / 4 + 256) {
+        q = it->second.first;
+        b = {it->first, it->second.second};
+        h->spares.erase(it);
+    } else {
+        const hipError_t e = pool_get(bytes, &q, &b.size, &b.device);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(FEHIP_EOOM, "hipMalloc of " + std::to_string(count * sizeof(P)) + " bytes failed: " +
+                                        hipGetErrorString(e));
+        }
     }
-    h->allocs.push_back(q);
+    h->allocs[q] = b;
     *ptr = (P *)q;
     return 0;
 }
@@ -216,9 +237,22 @@ static int dalloc_bytes(fehip_solver *h, void **ptr, size_t bytes) {
 
 static void dfree(fehip_solver *h, void *q) {
     if (!q) return;
-    auto it = std::find(h->allocs.begin(), h->allocs.end(), q);
-    if (it != h->allocs.end()) h->allocs.erase(it);
-    (void)hipFree(q);
+    auto it = h->allocs.find(q);
+    if (it == h->allocs.end()) return;
+    h->spares.emplace(it->second.size, std::make_pair(q, it->second.device));
+    h->allocs.erase(it);
+}
+
+// the handle's spare blocks go back to the pool; its stream must be idle
+static void release_spares(fehip_solver *h) {
+    for (auto &b : h->spares) pool_put(b.second.first, b.first, b.second.second);
+    h->spares.clear();
+}
+
+static void release_all(fehip_solver *h) {
+    for (auto &b : h->allocs) pool_put(b.first, b.second.size, b.second.device);
+    h->allocs.clear();
+    release_spares(h);
 }
 
 // integer tuning knob from the environment, clamped to [lo, hi]
@@ -725,8 +759,8 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
         bool armed = true;
         ~Cleanup() {
             if (!armed) return;
-            for (void *q : h->allocs) (void)hipFree(q);
-            h->allocs.clear();
+            if (h->stream) (void)hipStreamSynchronize(h->stream);
+            release_all(h);
             if (h->h_flag) (void)hipHostFree(h->h_flag);
             for (int e = 0; e < 2; e++)
                 if (h->poll_ev[e]) (void)hipEventDestroy(h->poll_ev[e]);
@@ -888,6 +922,7 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
         }
     }
     CHK(do_update_weights(h, weights));
+    release_spares(h);  // (do_update_weights ends with the stream idle)
     cleanup.armed = false;
     *out = hp.release();
     return 0;
@@ -1280,6 +1315,7 @@ static int get_plan(fehip_solver *h, int K, size_t ts, Plan **out, int64_t waves
         CHK(build_pieces(h, P, ts, dense_items, tiles_c));
     }
     HIPCHK(hipStreamSynchronize(h->stream));
+    release_spares(h);
     h->plans[key] = pl.release();
     *out = P;
     return 0;
@@ -4205,17 +4241,16 @@ void fehip_destroy(fehip_t *h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (auto &kv : h->plans) destroy_plan(h, kv.second);
     h->plans.clear();
-    for (void *q : h->allocs) (void)hipFree(q);
-    h->allocs.clear();
+    if (h->stream2) {
+        (void)hipStreamSynchronize(h->stream2);
+        (void)hipStreamDestroy(h->stream2);
+    }
+    release_all(h);
     if (h->h_flag) (void)hipHostFree(h->h_flag);
     for (int e = 0; e < 2; e++)
         if (h->poll_ev[e]) (void)hipEventDestroy(h->poll_ev[e]);
     if (h->fork_ev) (void)hipEventDestroy(h->fork_ev);
     if (h->join_ev) (void)hipEventDestroy(h->join_ev);
-    if (h->stream2) {
-        (void)hipStreamSynchronize(h->stream2);
-        (void)hipStreamDestroy(h->stream2);
-    }
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
 }
