@@ -667,14 +667,48 @@ static int compute_scale_cache(fehip_solver *h) {
     return 0;
 }
 
+__global__ void k_set_u64(unsigned long long *p, unsigned long long v) { *p = v; }
+
+// *bad = the first weight that is not positive and finite
+__global__ __launch_bounds__(kBlock) void k_bad_weight(const double *__restrict__ w, int64_t n,
+                                                       unsigned long long *bad) {
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
+        const double v = w[i];
+        if (!(v > 0.0 && v <= 1.7976931348623157e308)) {
+            atomicMin(bad, (unsigned long long)i);
+            break;
+        }
+    }
+}
+
 static int do_update_weights(fehip_solver *h, const double *w) {
     if (w) {
-        for (int64_t i = 0; i < h->N; i++)
-            if (!(w[i] > 0.0) || !std::isfinite(w[i]))
-                return fail(FEHIP_EARG, "weights must be positive and finite (observation " + std::to_string(i + 1) +
+        // into a block of its own: the handle stays as it is if they are refused
+        double *dw = nullptr;
+        unsigned long long *dbad = nullptr, bad = ~0ull;
+        CHK(dalloc(h, &dw, h->N));
+        int rc = dalloc(h, &dbad, 1);
+        auto check = [&]() -> int {
+            HIPCHK(copy_in(dw, w, sizeof(double) * h->N, h->stream));
+            hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, h->stream, dbad, ~0ull);
+            hipLaunchKernelGGL(k_bad_weight, dim3(std::min(grid_for(h->N, 4 * kBlock), 4096u)), dim3(kBlock), 0,
+                               h->stream, (const double *)dw, h->N, dbad);
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipMemcpyAsync(&bad, dbad, sizeof(bad), hipMemcpyDeviceToHost, h->stream));
+            HIPCHK(hipStreamSynchronize(h->stream));
+            if (bad != ~0ull)
+                return fail(FEHIP_EARG, "weights must be positive and finite (observation " + std::to_string(bad + 1) +
                                             ")");
-        if (!h->w_orig) CHK(dalloc(h, &h->w_orig, h->N));
-        HIPCHK(hipMemcpyAsync(h->w_orig, w, sizeof(double) * h->N, hipMemcpyHostToDevice, h->stream));
+            return 0;
+        };
+        if (rc == 0) rc = check();
+        dfree(h, dbad);
+        if (rc) {
+            dfree(h, dw);
+            return rc;
+        }
+        dfree(h, h->w_orig);
+        h->w_orig = dw;
     } else {
         dfree(h, h->w_orig);
         dfree(h, h->sqrtw_int);
@@ -780,9 +814,18 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
     std::vector<int32_t *> ref_orig(G, nullptr);
     {
         R *tmp = nullptr;
-        CHK(dalloc(h, &tmp, N));
         for (int g = 0; g < G; g++) {
             CHK(dalloc(h, &ref_orig[g], N));
+            bool bad = false;
+            hipError_t e = hipSuccess;
+            if (copy_in_refs(ref_orig[g], refs[g], N, h->n[g], &bad, h->stream, &e)) {
+                HIPCHK(e);
+                if (bad)
+                    return fail(FEHIP_EREF, "refs[" + std::to_string(g) + "] has a value outside 1.." +
+                                                std::to_string(h->n[g]));
+                continue;
+            }
+            if (!tmp) CHK(dalloc(h, &tmp, N));
             HIPCHK(hipMemcpyAsync(tmp, refs[g], sizeof(R) * N, hipMemcpyHostToDevice, h->stream));
             hipLaunchKernelGGL(k_refs_to_i32<R>, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, h->stream, tmp, N,
                                h->n[g], ref_orig[g], h->d_flag);
@@ -879,7 +922,7 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
         FeInfo &f = h->fe[g];
         if (interaction && interaction[g]) {
             CHK(dalloc(h, &f.z_orig, N));
-            HIPCHK(hipMemcpyAsync(f.z_orig, interaction[g], sizeof(double) * N, hipMemcpyHostToDevice, h->stream));
+            HIPCHK(copy_in(f.z_orig, interaction[g], sizeof(double) * N, h->stream));
         }
         CHK(dalloc(h, &f.scale_d, f.n));
         for (int q = 0; q < 2; q++) {
@@ -3557,11 +3600,10 @@ static int group_keys(fehip_solver *h, int64_t N, int32_t ncols, const int64_t *
     std::vector<const int64_t *> dk(ncols);
     for (int c = 0; c < ncols; c++) {
         dk[c] = dkeys + (size_t)c * N;
-        HIPCHK(hipMemcpyAsync(dkeys + (size_t)c * N, keys[c], sizeof(int64_t) * N, hipMemcpyHostToDevice, h->stream));
+        HIPCHK(copy_in(dkeys + (size_t)c * N, keys[c], sizeof(int64_t) * N, h->stream));
     }
     CHK(group_keys_device(h->stream, gs, N, ncols, dk.data(), drefs, ngroups));
-    HIPCHK(hipMemcpyAsync(refs, drefs, sizeof(int64_t) * N, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
+    HIPCHK(copy_out(refs, drefs, sizeof(int64_t) * N, h->stream));
     return 0;
 }
 
@@ -3724,8 +3766,7 @@ int fehip_solve_residuals_panels_host(fehip_t *const *hs, int32_t npanels, doubl
         ld[i] = h->N;
         rc = dalloc(h, &dY[i], (size_t)h->N * K[i]);
         for (int32_t c = 0; c < K[i] && rc == 0; c++) {
-            const hipError_t e = hipMemcpyAsync(dY[i] + (int64_t)c * h->N, cols[i][c], sizeof(double) * h->N,
-                                                hipMemcpyHostToDevice, h->stream);
+            const hipError_t e = copy_in(dY[i] + (int64_t)c * h->N, cols[i][c], sizeof(double) * h->N, h->stream);
             if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
         }
     }
@@ -3733,8 +3774,7 @@ int fehip_solve_residuals_panels_host(fehip_t *const *hs, int32_t npanels, doubl
     for (int32_t i = 0; i < npanels && rc == 0; i++) {
         fehip_solver *h = hs[i];
         for (int32_t c = 0; c < K[i] && rc == 0; c++) {
-            const hipError_t e = hipMemcpyAsync(cols[i][c], dY[i] + (int64_t)c * h->N, sizeof(double) * h->N,
-                                                hipMemcpyDeviceToHost, h->stream);
+            const hipError_t e = copy_out(cols[i][c], dY[i] + (int64_t)c * h->N, sizeof(double) * h->N, h->stream);
             if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
         }
     }
@@ -3760,16 +3800,14 @@ int fehip_solve_residuals(fehip_t *h, double *const *cols, int32_t K, double tol
     for (int32_t c0 = 0; c0 < K && rc == 0; c0 += bw) {
         const int k = std::min<int32_t>(bw, K - c0);
         for (int c = 0; c < k && rc == 0; c++) {
-            hipError_t e = hipMemcpyAsync(dY + (int64_t)c * h->N, cols[c0 + c], sizeof(double) * h->N,
-                                          hipMemcpyHostToDevice, h->stream);
+            hipError_t e = copy_in(dY + (int64_t)c * h->N, cols[c0 + c], sizeof(double) * h->N, h->stream);
             if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
         }
         if (rc == 0)
             rc = solve_residuals_dev(h, dY, k, h->N, tol, maxiter, iters ? iters + c0 : nullptr,
                                      converged ? converged + c0 : nullptr);
         for (int c = 0; c < k && rc == 0; c++) {
-            hipError_t e = hipMemcpyAsync(cols[c0 + c], dY + (int64_t)c * h->N, sizeof(double) * h->N,
-                                          hipMemcpyDeviceToHost, h->stream);
+            hipError_t e = copy_out(cols[c0 + c], dY + (int64_t)c * h->N, sizeof(double) * h->N, h->stream);
             if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
         }
         if (rc == 0) {
@@ -3792,7 +3830,7 @@ int fehip_solve_coefficients(fehip_t *h, const double *y, double tol, int64_t ma
     CHK(dalloc(h, &dc, h->p));
     int rc = 0;
     {
-        hipError_t e = hipMemcpyAsync(dy, y, sizeof(double) * h->N, hipMemcpyHostToDevice, h->stream);
+        hipError_t e = copy_in(dy, y, sizeof(double) * h->N, h->stream);
         if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
     }
     if (rc == 0) rc = solve_coefficients_dev(h, dy, tol, maxiter, dc, iters, converged);
@@ -3817,7 +3855,7 @@ int fehip_solve_coefficients_full(fehip_t *h, const double *y, double tol, int64
     CHK(dalloc(h, &dc, h->p));
     int rc = 0;
     {
-        hipError_t e = hipMemcpyAsync(dy, y, sizeof(double) * h->N, hipMemcpyHostToDevice, h->stream);
+        hipError_t e = copy_in(dy, y, sizeof(double) * h->N, h->stream);
         if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
     }
     if (rc == 0) rc = solve_coefficients_dev(h, dy, tol, maxiter, dc, iters, converged);
@@ -3827,8 +3865,7 @@ int fehip_solve_coefficients_full(fehip_t *h, const double *y, double tol, int64
         if (!obs[g]) continue;
         rc = full_dev(h, dc, g, dy);
         if (rc) break;
-        hipError_t e = hipMemcpyAsync(obs[g], dy, sizeof(double) * h->N, hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        const hipError_t e = copy_out(obs[g], dy, sizeof(double) * h->N, h->stream);
         if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
     }
     if (rc == 0 && coef) rc = s_block_to_caller(h, dc);
@@ -3923,7 +3960,7 @@ int fehip_features(fehip_t *h, const double *y, float *feats, double *coef_ap, d
     CHK(dalloc(h, &dy, h->N));
     CHK(dalloc(h, &dca, h->p));
     int rc = 0;
-    hipError_t e = hipMemcpyAsync(dy, y, sizeof(double) * h->N, hipMemcpyHostToDevice, h->stream);
+    hipError_t e = copy_in(dy, y, sizeof(double) * h->N, h->stream);
     if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
     const int prec = h->precision == FEHIP_MIXED ? FEHIP_FP64 : h->precision;
     if (rc == 0)
@@ -3965,8 +4002,7 @@ static int solve_from_common(fehip_t *h, double *const *cols, int32_t K, double 
     CHK(dalloc(h, &dY, (size_t)h->N * K));
     int rc = 0;
     for (int c = 0; c < K && rc == 0; c++) {
-        hipError_t e = hipMemcpyAsync(dY + (int64_t)c * h->N, cols[c], sizeof(double) * h->N, hipMemcpyHostToDevice,
-                                      h->stream);
+        hipError_t e = copy_in(dY + (int64_t)c * h->N, cols[c], sizeof(double) * h->N, h->stream);
         if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
     }
     const int prec = h->precision == FEHIP_MIXED ? FEHIP_FP64 : h->precision;
@@ -3975,8 +4011,7 @@ static int solve_from_common(fehip_t *h, double *const *cols, int32_t K, double 
             return decltype(eng)::solve_residuals_from(h, dY, K, h->N, tol, maxiter, coef0, net, iters, converged);
         });
     for (int c = 0; c < K && rc == 0; c++) {
-        hipError_t e = hipMemcpyAsync(cols[c], dY + (int64_t)c * h->N, sizeof(double) * h->N, hipMemcpyDeviceToHost,
-                                      h->stream);
+        hipError_t e = copy_out(cols[c], dY + (int64_t)c * h->N, sizeof(double) * h->N, h->stream);
         if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
     }
     if (rc == 0) {
@@ -4022,7 +4057,7 @@ int fehip_solve_coefficients_x0(fehip_t *h, const double *y, double tol, int64_t
     CHK(dalloc(h, &dy, h->N));
     CHK(dalloc(h, &dc, h->p));
     int rc = 0;
-    hipError_t e = hipMemcpyAsync(dy, y, sizeof(double) * h->N, hipMemcpyHostToDevice, h->stream);
+    hipError_t e = copy_in(dy, y, sizeof(double) * h->N, h->stream);
     if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
     const int prec = h->precision == FEHIP_MIXED ? FEHIP_FP64 : h->precision;
     FwlScope fwl(h);
