@@ -470,7 +470,7 @@ static int renumber_s(fehip_solver *h, int32_t *ref_s, const int32_t *ref_t, int
 // caller order -- the reference's summation order (:81-83) -- in double,
 // rounded into T after every add exactly as the Julia promotion does.
 // Levels with more than kScaleBig observations are left to k_scale_big.
-constexpr int32_t kScaleBig = 2048;
+constexpr int32_t kScaleBig = 128;
 
 template <typename T>
 __global__ void k_scale(const int32_t *__restrict__ off, const int32_t *__restrict__ perm, int64_t nlev,
@@ -503,6 +503,14 @@ __global__ void k_scale(const int32_t *__restrict__ off, const int32_t *__restri
         s = (T)((double)s + (zi * zi) * wi);
     }
     const T r = s > (T)0 ? (T)1 / (T)sqrt((double)s) : (T)0;
+    if (!w && !z) {
+        // a sum of ones, one after another: their count (a float stays at 2^24)
+        const int32_t n = sizeof(T) == 4 && q1 - q > (1 << 24) ? 1 << 24 : q1 - q;
+        const T s1 = (T)n, r = n > 0 ? (T)1 / (T)sqrt((double)s1) : (T)0;
+        scale_T[k] = r;
+        scale_d[k] = (double)r;
+        return;
+    }
     scale_T[k] = r;
     scale_d[k] = (double)r;
 }
@@ -517,8 +525,8 @@ __global__ __launch_bounds__(kWave) void k_scale_big(const int32_t *__restrict__
                                                      const double *__restrict__ z, T *__restrict__ scale_T,
                                                      double *__restrict__ scale_d) {
 #pragma clang fp contract(off)
-    constexpr int B = 16, CH = kWave * B;
-    __shared__ double buf[CH];
+    constexpr int B = 16, CH = kWave * B, A = 16;
+    __shared__ double buf[CH + 2 * A];
     const int lane = threadIdx.x;
     const int32_t k = levels[blockIdx.x];
     const int32_t q0 = off[k], q1 = off[k + 1];
@@ -545,7 +553,21 @@ __global__ __launch_bounds__(kWave) void k_scale_big(const int32_t *__restrict__
         if (base + CH < q1) load(base + CH);
         if (lane == 0) {
             const int32_t n = q1 - base < CH ? q1 - base : CH;
-            for (int32_t e = 0; e < n; e++) s = (T)((double)s + buf[e]);
+            double x[A], y[A];
+#pragma unroll
+            for (int j = 0; j < A; j++) x[j] = buf[j];
+            int32_t e = 0;
+            for (; e + 2 * A <= n; e += 2 * A) {
+#pragma unroll
+                for (int j = 0; j < A; j++) y[j] = buf[e + A + j];
+#pragma unroll
+                for (int j = 0; j < A; j++) s = (T)((double)s + x[j]);
+#pragma unroll
+                for (int j = 0; j < A; j++) x[j] = buf[e + 2 * A + j];  // (past the last chunk's end: not added)
+#pragma unroll
+                for (int j = 0; j < A; j++) s = (T)((double)s + y[j]);
+            }
+            for (; e < n; e++) s = (T)((double)s + buf[e]);
         }
         __syncthreads();
     }
@@ -564,6 +586,7 @@ __global__ void k_cache(const int32_t *__restrict__ perm_s, int64_t N, const int
 #pragma clang fp contract(off)
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= N) return;
+            // the next A terms are read from LDS while these are added
     const int32_t i = perm_s[j];
     const double zi = z ? z[i] : 1.0;
     const double wi = w ? w[i] : 1.0;
@@ -630,7 +653,7 @@ static int compute_scale_cache(fehip_solver *h) {
         hipLaunchKernelGGL(k_scale<T>, dim3(grid_for(f.n, 64)), dim3(64), 0, h->stream, f.ooff, f.operm, f.n,
                            h->w_orig, f.z_orig, (T *)f.scale_T[q], f.scale_d);
         HIPCHK(hipGetLastError());
-        if (f.big_levels.empty()) continue;
+        if (f.big_levels.empty() || (!h->w_orig && !f.z_orig)) continue;
         if (!f.d_big) {
             CHK(dalloc(h, &f.d_big, f.big_levels.size()));
             HIPCHK(hipMemcpyAsync(f.d_big, f.big_levels.data(), sizeof(int32_t) * f.big_levels.size(),
