@@ -372,32 +372,28 @@ static int csr_products(fehip_solver *h, const int32_t *skeys, int64_t N, int64_
 }
 
 
-// FE s's internal numbering: its levels ordered by their main level of FE t
-// (the t level holding the longest run of the s level's observations, ties
-// to the smaller t; levels without observations last), then by caller
-// number.  Workers sharing a main firm are then adjacent in the internal
+// FE s's internal numbering: its levels ordered by size class, then by their
+// main level of FE t (the t level holding the longest run of the s level's
+// observations, ties to the smaller t; levels without observations last), then
+// by caller number (k_main_level).  Workers sharing a main firm are then adjacent in the internal
 // order, so a firm's pieces lie close together in the piece order and the
 // piece launch's gathers of their sums share cache lines.  ref_s (the
-// caller's order, 0-based) is relabeled in place.
-static int renumber_s(fehip_solver *h, int32_t *ref_s, const int32_t *ref_t, int t) {
+// caller's order, 0-based) is relabeled in place.  perm_t: the observations
+// sorted by FE t.
+static int renumber_s(fehip_solver *h, int32_t *ref_s, const int32_t *ref_t, int t, const int32_t *perm_t) {
     const int64_t N = h->N, ns = h->n[h->s], nt = h->n[t];
-    int32_t *sk = nullptr, *p2 = nullptr, *k1 = nullptr, *ss = nullptr, *perm = nullptr, *tt = nullptr;
-    CHK(dalloc(h, &sk, N));
-    CHK(dalloc(h, &p2, N));
+    int32_t *k1 = nullptr, *ss = nullptr, *perm = nullptr, *tt = nullptr;
     CHK(dalloc(h, &k1, N));
     CHK(dalloc(h, &ss, N));
     CHK(dalloc(h, &perm, N));
     CHK(dalloc(h, &tt, N));
     // observations sorted by (s, t)
-    CHK(radix_sort(h, ref_t, N, nt, sk, p2));
-    hipLaunchKernelGGL(k_gather_perm<int32_t>, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, h->stream, ref_s, p2, N,
-                       k1);
-    CHK(radix_sort(h, k1, N, ns, ss, perm, p2));
+    hipLaunchKernelGGL(k_gather_perm<int32_t>, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, h->stream, ref_s, perm_t,
+                       N, k1);
+    CHK(radix_sort(h, k1, N, ns, ss, perm, perm_t));
     hipLaunchKernelGGL(k_gather_perm<int32_t>, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, h->stream, ref_t, perm, N,
                        tt);
     HIPCHK(hipGetLastError());
-    dfree(h, sk);
-    dfree(h, p2);
     dfree(h, k1);
     dfree(h, perm);
     // runs of one (s, t) pair
@@ -443,7 +439,7 @@ static int renumber_s(fehip_solver *h, int32_t *ref_s, const int32_t *ref_t, int
     hipLaunchKernelGGL(k_main_level, dim3(grid_for(ns, kBlock)), dim3(kBlock), 0, h->stream, (const int32_t *)roff,
                        (const int32_t *)run_start, (const int32_t *)run_t, ns, (int32_t)nt, mainl);
     HIPCHK(hipGetLastError());
-    CHK(radix_sort(h, mainl, ns, nt + 1, skeys, h->s_ext_of));
+    CHK(radix_sort(h, mainl, ns, kMainClasses * (nt + 1), skeys, h->s_ext_of));
     hipLaunchKernelGGL(k_invert_perm, dim3(grid_for(ns, kBlock)), dim3(kBlock), 0, h->stream,
                        (const int32_t *)h->s_ext_of, ns, h->s_int_of);
     hipLaunchKernelGGL(k_relabel, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, h->stream, ref_s, N,
@@ -870,7 +866,8 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
         if (g != h->s && h->n[g] > dense_limit(precision) && (t_sec < 0 || h->n[g] > h->n[t_sec])) t_sec = g;
     h->t_sec = t_sec;
     // FE s in its internal numbering from here on (FEHIP_RENUMBER=0 keeps the caller's)
-    if (t_sec >= 0 && env_int("FEHIP_RENUMBER", 1, 0, 1)) CHK(renumber_s(h, ref_orig[h->s], ref_orig[t_sec], t_sec));
+    if (t_sec >= 0 && h->n[t_sec] < INT32_MAX / kMainClasses - 1 && env_int("FEHIP_RENUMBER", 1, 0, 1))
+        CHK(renumber_s(h, ref_orig[h->s], ref_orig[t_sec], t_sec, t_perm));
     {
         FeInfo &f = h->fe[h->s];
         f.n = h->n[h->s];
@@ -880,18 +877,12 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
         CHK(dalloc(h, &h->ident, N));
         hipLaunchKernelGGL(k_iota, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, h->stream, h->ident, N);
         if (t_sec >= 0) {
-            int32_t *sk = nullptr, *p2 = nullptr, *k1 = nullptr;
-            CHK(dalloc(h, &sk, N));
-            CHK(dalloc(h, &p2, N));
+            int32_t *k1 = nullptr;
             CHK(dalloc(h, &k1, N));
-            CHK(radix_sort(h, ref_orig[t_sec], N, h->n[t_sec], sk, p2));
             hipLaunchKernelGGL(k_gather_perm<int32_t>, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, h->stream,
-                               ref_orig[h->s], p2, N, k1);
+                               ref_orig[h->s], (const int32_t *)t_perm, N, k1);
             HIPCHK(hipGetLastError());
-            CHK(radix_sort(h, k1, N, f.n, f.ref_int, h->perm_s, p2));
-            HIPCHK(hipStreamSynchronize(h->stream));
-            dfree(h, sk);
-            dfree(h, p2);
+            CHK(radix_sort(h, k1, N, f.n, f.ref_int, h->perm_s, t_perm));
             dfree(h, k1);
         } else {
             CHK(radix_sort(h, ref_orig[h->s], N, f.n, f.ref_int, h->perm_s));
@@ -922,11 +913,16 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
                            ref_orig[g], h->perm_s, N, f.ref_int);
         HIPCHK(hipGetLastError());
         // bucketing over the caller's order (bit-exact with bucketize_refs; used by scale!)
-        CHK(dalloc(h, &f.operm, N));
         CHK(dalloc(h, &f.ooff, f.n + 1));
         int32_t *skeys = nullptr;
-        CHK(dalloc(h, &skeys, N));
-        CHK(radix_sort(h, ref_orig[g], N, f.n, skeys, f.operm));
+        if (g == t_sec) {
+            skeys = t_keys;
+            f.operm = t_perm;
+        } else {
+            CHK(dalloc(h, &f.operm, N));
+            CHK(dalloc(h, &skeys, N));
+            CHK(radix_sort(h, ref_orig[g], N, f.n, skeys, f.operm));
+        }
         CHK(csr_products(h, skeys, N, f.n, f.ooff, nullptr));
         if (f.kind == KIND_CSR) {
             // bucketing over the internal order (locality of the D'u reads)
@@ -940,6 +936,14 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
     }
     for (int g = 0; g < G; g++) dfree(h, ref_orig[g]);
     free_sort_scratch(h);
+    // the observations sorted by FE t: for the numbering and the order below,
+    // and FE t's bucketing
+    int32_t *t_keys = nullptr, *t_perm = nullptr;
+    if (t_sec >= 0) {
+        CHK(dalloc(h, &t_keys, N));
+        CHK(dalloc(h, &t_perm, N));
+        CHK(radix_sort(h, ref_orig[t_sec], N, h->n[t_sec], t_keys, t_perm));
+    }
     // interactions (caller's order), scales and caches
     for (int g = 0; g < G; g++) {
         FeInfo &f = h->fe[g];
