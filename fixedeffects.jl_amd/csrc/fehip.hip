@@ -479,6 +479,14 @@ __global__ void k_scale(const int32_t *__restrict__ off, const int32_t *__restri
     T s = (T)0;
     const int32_t q1 = off[k + 1];
     int32_t q = off[k];
+    if (!w && !z) {
+        // a sum of ones, one after another: their count (a float stays at 2^24)
+        const int32_t n = sizeof(T) == 4 && q1 - q > (1 << 24) ? 1 << 24 : q1 - q;
+        const T s1 = (T)n, r = n > 0 ? (T)1 / (T)sqrt((double)s1) : (T)0;
+        scale_T[k] = r;
+        scale_d[k] = (double)r;
+        return;
+    }
     if (q1 - q > kScaleBig) return;
     for (; q + B <= q1; q += B) {
         double t[B];
@@ -499,14 +507,6 @@ __global__ void k_scale(const int32_t *__restrict__ off, const int32_t *__restri
         s = (T)((double)s + (zi * zi) * wi);
     }
     const T r = s > (T)0 ? (T)1 / (T)sqrt((double)s) : (T)0;
-    if (!w && !z) {
-        // a sum of ones, one after another: their count (a float stays at 2^24)
-        const int32_t n = sizeof(T) == 4 && q1 - q > (1 << 24) ? 1 << 24 : q1 - q;
-        const T s1 = (T)n, r = n > 0 ? (T)1 / (T)sqrt((double)s1) : (T)0;
-        scale_T[k] = r;
-        scale_d[k] = (double)r;
-        return;
-    }
     scale_T[k] = r;
     scale_d[k] = (double)r;
 }
@@ -548,6 +548,7 @@ __global__ __launch_bounds__(kWave) void k_scale_big(const int32_t *__restrict__
         __syncthreads();
         if (base + CH < q1) load(base + CH);
         if (lane == 0) {
+            // the next A terms are read from LDS while these are added
             const int32_t n = q1 - base < CH ? q1 - base : CH;
             double x[A], y[A];
 #pragma unroll
@@ -582,7 +583,6 @@ __global__ void k_cache(const int32_t *__restrict__ perm_s, int64_t N, const int
 #pragma clang fp contract(off)
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= N) return;
-            // the next A terms are read from LDS while these are added
     const int32_t i = perm_s[j];
     const double zi = z ? z[i] : 1.0;
     const double wi = w ? w[i] : 1.0;
@@ -865,6 +865,14 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
     for (int g = 0; g < G; g++)
         if (g != h->s && h->n[g] > dense_limit(precision) && (t_sec < 0 || h->n[g] > h->n[t_sec])) t_sec = g;
     h->t_sec = t_sec;
+    // the observations sorted by FE t: for the numbering and the order below,
+    // and FE t's bucketing
+    int32_t *t_keys = nullptr, *t_perm = nullptr;
+    if (t_sec >= 0) {
+        CHK(dalloc(h, &t_keys, N));
+        CHK(dalloc(h, &t_perm, N));
+        CHK(radix_sort(h, ref_orig[t_sec], N, h->n[t_sec], t_keys, t_perm));
+    }
     // FE s in its internal numbering from here on (FEHIP_RENUMBER=0 keeps the caller's)
     if (t_sec >= 0 && h->n[t_sec] < INT32_MAX / kMainClasses - 1 && env_int("FEHIP_RENUMBER", 1, 0, 1))
         CHK(renumber_s(h, ref_orig[h->s], ref_orig[t_sec], t_sec, t_perm));
@@ -936,14 +944,6 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
     }
     for (int g = 0; g < G; g++) dfree(h, ref_orig[g]);
     free_sort_scratch(h);
-    // the observations sorted by FE t: for the numbering and the order below,
-    // and FE t's bucketing
-    int32_t *t_keys = nullptr, *t_perm = nullptr;
-    if (t_sec >= 0) {
-        CHK(dalloc(h, &t_keys, N));
-        CHK(dalloc(h, &t_perm, N));
-        CHK(radix_sort(h, ref_orig[t_sec], N, h->n[t_sec], t_keys, t_perm));
-    }
     // interactions (caller's order), scales and caches
     for (int g = 0; g < G; g++) {
         FeInfo &f = h->fe[g];
