@@ -686,6 +686,8 @@ static int compute_scale_cache(fehip_solver *h) {
     return 0;
 }
 
+static void drop_graphs(fehip_solver *h);
+
 __global__ void k_set_u64(unsigned long long *p, unsigned long long v) { *p = v; }
 
 // *bad = the first weight that is not positive and finite
@@ -701,6 +703,8 @@ __global__ __launch_bounds__(kBlock) void k_bad_weight(const double *__restrict_
 }
 
 static int do_update_weights(fehip_solver *h, const double *w) {
+    // the captured passes over the observations hold sqrt(w)'s address, or none
+    if ((w != nullptr) != (h->w_orig != nullptr)) drop_graphs(h);
     if (w) {
         // into a block of its own: the handle stays as it is if they are refused
         double *dw = nullptr;
@@ -1628,6 +1632,13 @@ static void destroy_plan(fehip_solver *h, Plan *P) {
     for (void *q : ptrs) dfree(h, q);
     destroy_pieces(h, P->pc);
     delete P;
+}
+
+static void drop_graphs(fehip_solver *h) {
+    for (auto &kv : h->plans) {
+        if (kv.second->graph) (void)hipGraphExecDestroy(kv.second->graph);
+        kv.second->graph = nullptr;
+    }
 }
 
 static void destroy_all_plans(fehip_solver *h) {
