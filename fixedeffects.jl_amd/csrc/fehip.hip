@@ -3553,8 +3553,9 @@ __global__ void k_minmax_init(long long *mm) {
     }
 }
 
+// dense[i] = base + the rank of u[i] among its distinct values
 static int number_keys(hipStream_t st, GroupScratch &gs, const uint64_t *u, int64_t n, int bits, int64_t *dense,
-                       int64_t *ngroups) {
+                       int64_t base, int64_t *ngroups) {
     const int passes = std::max(1, (bits + 7) / 8);
     const uint64_t *kin = u;
     const int32_t *vin = nullptr;
@@ -3575,7 +3576,7 @@ static int number_keys(hipStream_t st, GroupScratch &gs, const uint64_t *u, int6
     hipLaunchKernelGGL(k_group_heads, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, st, kin, n, gs.flag);
     CHK(exclusive_scan_u32(st, gs.flag, n, gs.ex, true, gs.sums2));
     hipLaunchKernelGGL(k_group_assign, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, st, (const uint32_t *)gs.ex,
-                       (const uint32_t *)gs.flag, vin, n, dense);
+                       (const uint32_t *)gs.flag, vin, n, base, dense);
     HIPCHK(hipGetLastError());
     uint32_t total = 0;
     HIPCHK(hipMemcpyAsync(&total, gs.ex + n, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
@@ -3594,19 +3595,39 @@ static int bits_of(uint64_t range) {
 // (N int64, 1-based), with every buffer taken from gs; on stream st.
 static int group_keys_device(hipStream_t st, GroupScratch &gs, int64_t N, int32_t ncols,
                              const int64_t *const *dkeys, int64_t *drefs, int64_t *ngroups) {
-    int64_t n_prev = 0;
+    std::vector<long long> lo(ncols);
+    std::vector<int> bits(ncols);
+    int total = 0;
     for (int c = 0; c < ncols; c++) {
-        hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, st, gs.mm);
-        hipLaunchKernelGGL(k_minmax_i64, dim3((unsigned)std::min<int64_t>(grid_for(N, kBlock), 4096)), dim3(kBlock),
-                           0, st, dkeys[c], N, gs.mm);
         long long hm[2];
+        hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, st, gs.mm);
+        hipLaunchKernelGGL(k_minmax_i64, dim3((unsigned)std::min<int64_t>(grid_for(N, kBlock), 1024)), dim3(kBlock),
+                           0, st, dkeys[c], N, gs.mm);
         HIPCHK(hipMemcpyAsync(hm, gs.mm, sizeof(hm), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
-        hipLaunchKernelGGL(k_key_offset, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, st, dkeys[c], N, (int64_t)hm[0],
-                           gs.u);
+        lo[c] = hm[0];
+        bits[c] = bits_of((uint64_t)hm[1] - (uint64_t)hm[0]);
+        total += bits[c];
+    }
+    auto offset = [&](int c, int shift, uint64_t *u) {
+        hipLaunchKernelGGL(k_key_offset, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, st, dkeys[c], N, (int64_t)lo[c],
+                           shift, u);
+    };
+    int64_t n_prev = 0;
+    if (total <= 64) {
+        // every column's offset in one word, the first in the top bits: their
+        // order is the lexicographic one, and one sort of ceil(total / 8)
+        // passes numbers the combinations (two columns of 23 and 19 bits, N =
+        // 1e7: 6 passes and one numbering instead of 11 and three)
+        for (int c = 0; c < ncols; c++) offset(c, c ? bits[c] : -1, gs.u);
+        CHK(number_keys(st, gs, gs.u, N, total, drefs, 1, &n_prev));
+        *ngroups = n_prev;
+        return 0;
+    }
+    for (int c = 0; c < ncols; c++) {
+        offset(c, -1, gs.u);
         int64_t nc = 0;
-        CHK(number_keys(st, gs, gs.u, N, bits_of((uint64_t)hm[1] - (uint64_t)hm[0]), c == 0 ? gs.dense : gs.dcol,
-                        &nc));
+        CHK(number_keys(st, gs, gs.u, N, bits[c], c == 0 ? gs.dense : gs.dcol, 0, &nc));
         if (c == 0) {
             n_prev = nc;
             continue;
@@ -3614,7 +3635,7 @@ static int group_keys_device(hipStream_t st, GroupScratch &gs, int64_t N, int32_
         // combinations of distinct values: n_prev * nc <= N * N < 2^63
         hipLaunchKernelGGL(k_group_combine, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, st,
                            (const int64_t *)gs.dense, (const int64_t *)gs.dcol, N, nc, gs.u);
-        CHK(number_keys(st, gs, gs.u, N, bits_of((uint64_t)(n_prev * nc - 1)), gs.dense, &n_prev));
+        CHK(number_keys(st, gs, gs.u, N, bits_of((uint64_t)(n_prev * nc - 1)), gs.dense, 0, &n_prev));
     }
     hipLaunchKernelGGL(k_plus_one, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, st, (const int64_t *)gs.dense, N,
                        drefs);
