@@ -39,6 +39,7 @@
 #include "fehip_common.h"
 #include "hostmem.h"
 #include "linmap.h"
+#include "normal.h"
 
 using namespace fehip;
 
@@ -190,6 +191,11 @@ struct fehip_solver {
     int32_t *cc_nodes = nullptr;  // p
     int32_t *cc_start = nullptr;  // p + 2
     uint32_t *cc_ncomp = nullptr; // 1
+    // level-space form of the FP64 iteration (normal.h), built at the first
+    // solve: 0 not looked at, 1 built, -1 not taken (FEHIP_NORMAL=0, or too
+    // many entries)
+    NormalMat nf;
+    int nf_state = 0;
 };
 
 // With separate CSR and fix-up launches (FEHIP_SEG_FIX=0), from this batch
@@ -340,6 +346,21 @@ static int radix_sort(fehip_solver *h, const int32_t *keys, int64_t N, int64_t n
     }
     return 0;
 }
+
+namespace fehip {
+// what the construction of the normal matrix (normal.hip) uses of the solver
+int solver_alloc(fehip_solver *h, void **ptr, size_t bytes) { return dalloc_bytes(h, ptr, bytes); }
+void solver_free(fehip_solver *h, void *ptr) { dfree(h, ptr); }
+int solver_sort(fehip_solver *h, const int32_t *keys, int64_t n, int64_t nlev, int32_t *keys_out, int32_t *vals_out,
+                const int32_t *vals_in) {
+    return radix_sort(h, keys, n, nlev, keys_out, vals_out, vals_in);
+}
+// exclusive scan with the total in out[n]
+int solver_scan(fehip_solver *h, const uint32_t *in, int64_t n, uint32_t *out) {
+    CHK(ensure_sort_scratch(h, n));  // (its chunk sums cover 256 n entries / kSortTile)
+    return exclusive_scan_u32(h, in, n, out, true, h->sums);
+}
+}  // namespace fehip
 
 // offsets, head bits, word prefix and segment->level map of a sorted key array
 static int csr_products(fehip_solver *h, const int32_t *skeys, int64_t N, int64_t nlev, int32_t *off,
@@ -686,6 +707,7 @@ static int compute_scale_cache(fehip_solver *h) {
     return 0;
 }
 
+static int refresh_normal(fehip_solver *h);
 static void drop_graphs(fehip_solver *h);
 
 __global__ void k_set_u64(unsigned long long *p, unsigned long long v) { *p = v; }
@@ -741,6 +763,7 @@ static int do_update_weights(fehip_solver *h, const double *w) {
     }
     if (h->precision == FEHIP_FP32) return compute_scale_cache<float>(h);
     CHK(compute_scale_cache<double>(h));
+    CHK(refresh_normal(h));
     if (h->precision == FEHIP_MIXED) {
         // the FP32 streams hold the FP64 scales and caches rounded once
         for (int g = 0; g < h->G; g++) {
@@ -760,6 +783,47 @@ static int do_update_weights(fehip_solver *h, const double *w) {
         CHK(set_sqrtw_T(h, 1));
         HIPCHK(hipStreamSynchronize(h->stream));
     }
+    return 0;
+}
+
+// ---------------------------------------------------------------------------
+// the level-space form of the iteration
+// ---------------------------------------------------------------------------
+static NfInput nf_input(const fehip_solver *h) {
+    NfInput in;
+    in.N = h->N;
+    in.G = h->G;
+    in.s = h->s;
+    in.t_sec = h->t_sec;
+    in.n = h->n.data();
+    in.off = h->off.data();
+    for (int g = 0; g < h->G; g++) {
+        in.ref[g] = h->fe[g].ref_int;
+        in.cache[g] = (const double *)h->fe[g].cache_int[0];
+    }
+    in.stream = h->stream;
+    return in;
+}
+
+// the normal matrix follows new caches
+static int refresh_normal(fehip_solver *h) { return h->nf_state == 1 ? nf_values(nf_input(h), h->nf) : 0; }
+
+// Builds the normal matrix of an FP64 handle's fixed effects once
+static int ensure_normal(fehip_solver *h) {
+    if (h->nf_state) return 0;
+    h->nf_state = -1;
+    if (h->G < 2 || !h->has64 || !env_int("FEHIP_NORMAL", 1, 0, 1)) return 0;
+    int fits = 0;
+    const NfInput in = nf_input(h);
+    const int rc = nf_build(h, in, 6 * h->N, h->nf, &fits);
+    free_sort_scratch(h);
+    if (rc == FEHIP_EOOM) return 0;  // the passes over the observations need no more memory
+    CHK(rc);
+    if (!fits) return 0;
+    CHK(nf_values(in, h->nf));
+    HIPCHK(hipStreamSynchronize(h->stream));
+    release_spares(h);
+    h->nf_state = 1;
     return 0;
 }
 
@@ -1137,6 +1201,16 @@ struct Plan {
     void *zs = nullptr;
     ColOps *ops_one = nullptr, *ops_neg = nullptr, *ops_sub = nullptr;
     PieceForm pc;
+    // level-space iteration: M v, the vector that alternates with v as the
+    // current and the previous one, per-column coefficients, partials of
+    // v'Mv, ||x||^2 and the step's norm, and the parts of cut rows
+    double *nq = nullptr, *nw = nullptr;
+    NfCols *ncols = nullptr;
+    void *nstate = nullptr;      // the state's second copy (folded scalar steps)
+    bool nfold = false;
+    int final_copy = 0;          // where the last solve left its state
+    double *npa = nullptr, *npx = nullptr, *npw = nullptr, *nhead = nullptr, *ntail = nullptr;
+    unsigned nblocks = 0, nstep = 0, nfix = 0;
 };
 
 static int build_pieces(fehip_solver *h, Plan *P, size_t ts, const std::vector<FixItem> &dense_items,
@@ -1628,7 +1702,8 @@ static void destroy_plan(fehip_solver *h, Plan *P) {
     void *ptrs[] = {P->items, P->tileA, P->tileB, P->dpart, P->part_db, P->part_seg, P->part_fix, P->part_upd,
                     P->part_fused, P->wsum, P->sdirect, P->vt, P->state, P->ops_db, P->ops_dtx, P->ops_once, P->all_done, P->u, P->r, P->x,
                     P->v, P->hh, P->hbar, P->dY, P->tstart, P->items_s, P->items_o, P->items_sd, P->items_c,
-                    P->zs, P->ops_one, P->ops_neg, P->ops_sub, P->items_d};
+                    P->zs, P->ops_one, P->ops_neg, P->ops_sub, P->items_d, P->nq, P->nw, P->ncols, P->npa, P->npx,
+                    P->npw, P->nhead, P->ntail, P->nstate};
     for (void *q : ptrs) dfree(h, q);
     destroy_pieces(h, P->pc);
     delete P;
@@ -2774,8 +2849,106 @@ struct Engine {
         update(h, P);
     }
 
+    // the level-space iteration (normal.h) is in use: FP64 on a handle that has M
+    static bool use_nf(const fehip_solver *h, const Plan *P) { return sizeof(T) == 8 && h->nf_state == 1 && P->nq; }
+
+    static int nf_plan(fehip_solver *h, Plan *P) {
+        CHK(ensure_normal(h));
+        if (h->nf_state != 1 || P->nq) return 0;
+        const NormalMat &m = h->nf;
+        P->nblocks = nf_apply_blocks(K, m.ntile);
+        P->nfix = (unsigned)std::min(std::max(m.nitem, 1), 1024);
+        P->nstep = P->nfix + std::min(grid_for(h->p * K, 4 * kBlock), 1024u);
+        P->nfold = std::max(P->nblocks, P->nstep) * (int64_t)K <= kNfFold;
+        CHK(dalloc(h, &P->ncols, 2));
+        CHK(dalloc_bytes(h, &P->nstate, sizeof(LsmrState<double>) * K));
+        CHK(dalloc(h, &P->npa, (size_t)P->nblocks * K));
+        CHK(dalloc(h, &P->npx, (size_t)2 * P->nstep * K));
+        CHK(dalloc(h, &P->npw, (size_t)2 * P->nstep * K));
+        CHK(dalloc(h, &P->nhead, (size_t)m.ntile * K));
+        CHK(dalloc(h, &P->ntail, (size_t)m.ntile * K));
+        CHK(dalloc(h, &P->nw, (size_t)h->p * K));
+        CHK(dalloc(h, &P->nq, (size_t)h->p * K));
+        return 0;
+    }
+
+    // one LSMR iteration in level space; odd: the current vector is in nw
+    static void nf_iteration(fehip_solver *h, Plan *P, bool odd) {
+        const NormalMat &m = h->nf;
+        double *w = odd ? P->nw : (double *)P->v, *wold = odd ? (double *)P->v : P->nw;
+        NfApply a{};
+        a.off = m.off;
+        a.col = m.col;
+        a.val = m.val;
+        a.tile_e = m.tile_e;
+        a.tile_r = m.tile_r;
+        a.n0 = a.nt = m.ntile;
+        a.w = w;
+        a.q = P->nq;
+        a.pa = P->npa;
+        a.head = P->nhead;
+        a.tail = P->ntail;
+        a.all_done = P->all_done;
+        NfStep s{};
+        if (h->fwl_now) {
+            // FE s eliminated: its rows of M v first, negated in its (else
+            // zero) block of v; the other rows of M on that vector are then
+            // (I - A_s A_s') A_o in normal form
+            NfApply b = a;
+            b.t0 = m.ts0;
+            b.n0 = b.nt = m.ts1 - m.ts0;
+            b.neg = w;
+            nf_apply(K, b, P->nblocks, h->stream);
+            nf_fix_neg(K, m.items + m.is0, m.is1 - m.is0, P->nhead, P->ntail, w, P->all_done, h->stream);
+            a.n0 = m.ts0;
+            a.t1 = m.ts1;
+            a.nt = m.ntile - (m.ts1 - m.ts0);
+            s.row0 = h->off[h->s];
+            s.rown = h->n[h->s];
+        }
+        nf_apply(K, a, P->nblocks, h->stream);
+        // folded, the state, the coefficients and the step's partials alternate
+        // between two copies (the first is current when a solve begins)
+        const bool fold = P->nfold;
+        const size_t np = (size_t)P->nstep * K;
+        NfScalars c{};
+        c.pa = P->npa;
+        c.pw = P->npw + (fold && !odd ? np : 0);
+        c.px = P->npx + (fold && !odd ? np : 0);
+        c.na = (int32_t)P->nblocks;
+        c.nw = (int32_t)P->nstep;
+        c.sin = fold && odd ? P->nstate : P->state;
+        c.sout = fold && !odd ? P->nstate : P->state;
+        c.cin = P->ncols + (fold && odd);
+        c.cout = P->ncols + (fold && !odd);
+        c.copy = fold && !odd;
+        c.all_done = P->all_done;
+        if (fold) s.fold = c;
+        else nf_scalars(K, c, h->stream);
+        s.p = h->p;
+        s.q = P->nq;
+        s.w = w;
+        s.wold = wold;
+        s.h = (double *)P->hh;
+        s.hbar = (double *)P->hbar;
+        s.x = (double *)P->x;
+        s.cols = P->ncols;
+        s.items = m.items;
+        s.nitem = m.nitem;
+        s.split = m.split;
+        s.head = P->nhead;
+        s.tail = P->ntail;
+        s.pw = P->npw + (fold && odd ? np : 0);
+        s.px = P->npx + (fold && odd ? np : 0);
+        s.all_done = P->all_done;
+        s.fix_blocks = P->nfix;
+        nf_step(K, s, P->nstep, h->stream);
+    }
+
     static int ensure_graph(fehip_solver *h, Plan *P) {
-        const int M = h->poll_iters;
+        const bool nf = use_nf(h, P);
+        // (the level-space iterations alternate two vectors: an even number per graph)
+        const int M = nf ? (h->poll_iters + 1) / 2 * 2 : h->poll_iters;
         if (P->graph && P->graph_iters == M && P->graph_fwl == h->fwl_now) return 0;
         // the split fix-up's second stream exists only on handles whose graph
         // uses it: every stream of the process shares a few hardware queues,
@@ -2791,7 +2964,10 @@ struct Engine {
         }
         hipGraph_t g = nullptr;
         HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        for (int it = 0; it < M; it++) iteration(h, P);
+        for (int it = 0; it < M; it++) {
+            if (nf) nf_iteration(h, P, it & 1);
+            else iteration(h, P);
+        }
         hipError_t e = hipStreamEndCapture(h->stream, &g);
         if (e != hipSuccess) return fail(FEHIP_EHIP, std::string("graph capture failed: ") + hipGetErrorString(e));
         e = hipGraphInstantiate(&P->graph, g, nullptr, nullptr, 0);
@@ -2821,6 +2997,8 @@ struct Engine {
     }
 
     static int lsmr_start(fehip_solver *h, Plan *P, int Kreal, double tol, int64_t maxiter, Run &run) {
+        if constexpr (sizeof(T) == 8) CHK(nf_plan(h, P));
+        const bool nf = use_nf(h, P);
         hipLaunchKernelGGL((k_lsmr_setup<Tr>), dim3(1), dim3(64), 0, h->stream, (LsmrState<Tr> *)P->state, K, Kreal,
                            tol, tol, 1e8, maxiter, P->all_done);
         if (h->fwl_now) {
@@ -2850,10 +3028,14 @@ struct Engine {
         }
         hipLaunchKernelGGL((k_init_vectors<T, Tr, K>), dim3(P->upd_blocks), dim3(kBlock), 0, h->stream, h->p * K,
                            (T *)P->v, (T *)P->hh, (T *)P->hbar, (const void *)P->state,
-                           (const T *)h->scale_all[pidx<T>()], (T *)P->vt);
-        // the factored iteration with K < 8 keeps u as sqrt(w) .* u (not
-        // the piece form)
-        if (ut_now(h, P) && h->sqrtw_T[pidx<T>()])
+                           (const T *)h->scale_all[pidx<T>()], nf ? (T *)nullptr : (T *)P->vt);
+        if (nf) {
+            hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream, P->nw,
+                               h->p * K, 0.0);
+            nf_init_cols(K, P->state, P->ncols, h->stream);
+        } else if (ut_now(h, P) && h->sqrtw_T[pidx<T>()])
+            // the factored iteration with K < 8 keeps u as sqrt(w) .* u (not
+            // the piece form)
             hipLaunchKernelGGL(k_scale_rows<T>, dim3(grid_for(h->N * K, kBlock)), dim3(kBlock), 0, h->stream,
                                (T *)P->u, (const T *)h->sqrtw_T[pidx<T>()], h->N, K);
         HIPCHK(hipGetLastError());
@@ -2880,6 +3062,7 @@ struct Engine {
             if (q != hipSuccess) return fail(FEHIP_EHIP, std::string("event query: ") + hipGetErrorString(q));
         }
         if (h->h_flag[1 + run.cur]) {
+            P->final_copy = h->h_flag[1 + run.cur] - 1;
             HIPCHK(hipStreamSynchronize(h->stream));
             finished = true;
             return 0;
@@ -2944,7 +3127,8 @@ struct Engine {
     static int read_state(fehip_solver *h, Plan *P, int Kreal, std::vector<int64_t> &iters,
                           std::vector<int> &conv) {
         std::vector<LsmrState<Tr>> st(K);
-        HIPCHK(hipMemcpyAsync(st.data(), P->state, sizeof(LsmrState<Tr>) * K, hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(hipMemcpyAsync(st.data(), P->final_copy ? P->nstate : P->state, sizeof(LsmrState<Tr>) * K,
+                              hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
         h->last_info.assign((size_t)Kreal * 9, 0.0);
         for (int c = 0; c < Kreal; c++) {
@@ -3308,7 +3492,11 @@ struct Mixed {
 
     static int solve_residuals(fehip_solver *h, double *dY, int Kreal, int64_t ldY, double tol, int64_t maxiter,
                                int64_t *iters, uint8_t *converged) {
-        if (h->G == 1) return E64::solve_residuals(h, dY, Kreal, ldY, tol, maxiter, iters, converged);
+        // an FP64 iteration in level space takes less time than one over the
+        // FP32 streams, and the second phase would start its Krylov space anew
+        CHK(ensure_normal(h));
+        if (h->G == 1 || h->nf_state == 1)
+            return E64::solve_residuals(h, dY, Kreal, ldY, tol, maxiter, iters, converged);
         Plan *P32 = nullptr, *P64 = nullptr;
         CHK((get_plan_for<float, F32x2, K>(h, &P32)));
         CHK((get_plan_for<double, double, K>(h, &P64)));
@@ -3330,6 +3518,8 @@ struct Mixed {
 
     static int solve_coefficients(fehip_solver *h, double *dy, double tol, int64_t maxiter, double *dcoef,
                                   int64_t *iters, uint8_t *converged) {
+        CHK(ensure_normal(h));
+        if (h->nf_state == 1) return E64::solve_coefficients(h, dy, tol, maxiter, dcoef, iters, converged);
         Plan *P32 = nullptr, *P64 = nullptr;
         CHK((get_plan_for<float, F32x2, K>(h, &P32)));
         CHK((get_plan_for<double, double, K>(h, &P64)));

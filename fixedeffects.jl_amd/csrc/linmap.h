@@ -229,47 +229,11 @@ __device__ void fin_after_db(LsmrState<Tr> &s, double usq, int mode, int c, ColO
     }
 }
 
-// after v = A'u - beta v: alpha = ||v|| and the plane rotations (:67-98 at
-// set-up; :109-182 per iteration).  Leaves the h/hbar/x coefficients.
+// the plane rotations and estimates of one iteration, from alpha and beta
+// (:112-191)
 template <typename Tr>
-__device__ void fin_after_dtx(LsmrState<Tr> &s, double vsq, int mode, int c, ColOps *nx_db) {
+__device__ void fin_rotate(LsmrState<Tr> &s, int c, ColOps *nx_db) {
 #pragma clang fp contract(off)
-    if (s.done) {
-        nx_db->on[c] = 0;
-        return;
-    }
-    if (mode == MODE_INIT) {
-        const Tr alpha = (Tr)sqrt(vsq);
-        s.alpha = alpha;
-        s.inv_alpha = alpha > (Tr)0 ? (Tr)1 / alpha : (Tr)1;
-        s.zetabar = alpha * s.beta;
-        s.alphabar = alpha;
-        s.rho = 1; s.rhobar = 1; s.cbar = 1; s.sbar = 0;
-        s.betadd = s.beta; s.betad = 0; s.rhodold = 1; s.tautildeold = 0; s.thetatilde = 0;
-        s.zeta = 0; s.d = 0;
-        s.normA = -1; s.condA = -1; s.normx = -1;
-        s.normA2 = alpha * alpha;
-        s.maxrbar = 0;
-        s.minrbar = big_minrbar<Tr>();
-        s.normb = s.beta;
-        s.istop = 0;
-        s.normr = s.beta;
-        s.normAr = alpha * s.beta;
-        s.iter = 0;
-        s.vskip = 0;
-        if (s.normAr == (Tr)0 || s.maxiter <= 0) s.done = 1;  // :101-102
-        nx_db->a[c] = 1.0;
-        nx_db->b[c] = (double)(-(alpha * s.inv_beta));
-        nx_db->on[c] = s.done ? 0 : 1;
-        return;
-    }
-    if (!s.vskip) {
-        const Tr alpha = (Tr)sqrt(vsq);
-        s.alpha = alpha;
-        s.inv_alpha = alpha > (Tr)0 ? (Tr)1 / alpha : (Tr)1;
-    } else {
-        s.inv_alpha = (Tr)1;
-    }
     const Tr alpha = s.alpha, beta = s.beta, lambda = (Tr)0;
     // Qhat_{k,2k+1} (:114-116)
     const Tr alphahat = (Tr)sqrt((double)(s.alphabar * s.alphabar + lambda * lambda));
@@ -328,6 +292,50 @@ __device__ void fin_after_dtx(LsmrState<Tr> &s, double vsq, int mode, int c, Col
     nx_db->b[c] = (double)(-(s.alpha * s.inv_beta));
     nx_db->on[c] = 1;
     s.pending = 1;
+}
+
+// after v = A'u - beta v: alpha = ||v|| and the plane rotations (:67-98 at
+// set-up; :109-182 per iteration).  Leaves the h/hbar/x coefficients.
+template <typename Tr>
+__device__ void fin_after_dtx(LsmrState<Tr> &s, double vsq, int mode, int c, ColOps *nx_db) {
+#pragma clang fp contract(off)
+    if (s.done) {
+        nx_db->on[c] = 0;
+        return;
+    }
+    if (mode == MODE_INIT) {
+        const Tr alpha = (Tr)sqrt(vsq);
+        s.alpha = alpha;
+        s.inv_alpha = alpha > (Tr)0 ? (Tr)1 / alpha : (Tr)1;
+        s.zetabar = alpha * s.beta;
+        s.alphabar = alpha;
+        s.rho = 1; s.rhobar = 1; s.cbar = 1; s.sbar = 0;
+        s.betadd = s.beta; s.betad = 0; s.rhodold = 1; s.tautildeold = 0; s.thetatilde = 0;
+        s.zeta = 0; s.d = 0;
+        s.normA = -1; s.condA = -1; s.normx = -1;
+        s.normA2 = alpha * alpha;
+        s.maxrbar = 0;
+        s.minrbar = big_minrbar<Tr>();
+        s.normb = s.beta;
+        s.istop = 0;
+        s.normr = s.beta;
+        s.normAr = alpha * s.beta;
+        s.iter = 0;
+        s.vskip = 0;
+        if (s.normAr == (Tr)0 || s.maxiter <= 0) s.done = 1;  // :101-102
+        nx_db->a[c] = 1.0;
+        nx_db->b[c] = (double)(-(alpha * s.inv_beta));
+        nx_db->on[c] = s.done ? 0 : 1;
+        return;
+    }
+    if (!s.vskip) {
+        const Tr alpha = (Tr)sqrt(vsq);
+        s.alpha = alpha;
+        s.inv_alpha = alpha > (Tr)0 ? (Tr)1 / alpha : (Tr)1;
+    } else {
+        s.inv_alpha = (Tr)1;
+    }
+    fin_rotate<Tr>(s, c, nx_db);
 }
 
 // after the h/hbar/x update: ||x|| and the stopping rules (:192-215).

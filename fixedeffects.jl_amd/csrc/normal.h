@@ -1,0 +1,137 @@
+// normal.h -- the level-space form of the LSMR iteration: the normal matrix
+// M = A'A of the scaled fixed-effect map (unit diagonal) as one sparse matrix
+// over the levels, and the launches of an iteration that reads M instead of
+// the observations.
+#pragma once
+
+#include <vector>
+
+#include "fehip_common.h"
+
+struct fehip_solver;
+
+namespace fehip {
+
+// A tile is what one wave takes at a time: consecutive entries, and the rows
+// that begin among them.
+constexpr int kNfTile = 512;    // entries + kNfRow per row that a tile aims at
+constexpr int kNfSlack = 128;   // a row with at most this many units left at a tile's end is finished in it
+constexpr int kNfCap = kNfTile + kNfSlack;
+constexpr int kNfRow = 8;       // tile units of one row beside its entries (its vector elements)
+constexpr int kNfRows = kNfCap / kNfRow + 2;  // rows one tile owns, at most
+
+// a row whose entries lie in several tiles: [t0, t1) hold its later parts,
+// tile t0 - 1 its first
+struct NfItem {
+    int32_t row, t0, t1;
+};
+
+// cells (distinct level pairs) of one pair of FEs
+struct NfPair {
+    int a = 0, b = 0;              // cells sorted by (level of a, level of b)
+    int64_t ncell = 0;
+    int32_t *order = nullptr;      // internal positions sorted by (a, b); nullptr: the internal order itself
+    int32_t *start = nullptr;      // ncell + 1: first position (in that order) of each cell
+    int32_t *dsta = nullptr, *dstb = nullptr;  // the cell's entry in row a and in row b
+    int32_t *big = nullptr;        // cells of more than kNfBigCell observations
+    int32_t nbig = 0;
+};
+constexpr int kNfBigCell = 32;
+
+struct NormalMat {
+    int64_t p = 0, nnz = 0;
+    int32_t *off = nullptr, *col = nullptr;  // p + 1, nnz
+    double *val = nullptr;                   // nnz: sum over the cell of cache_a * cache_b
+    std::vector<NfPair> pairs;
+    // tiles: entries [e[k], e[k+1]), rows whose entries start in it [r[k], r[k+1])
+    int32_t ntile = 0, ts0 = 0, ts1 = 0;     // [ts0, ts1): the tiles of FE s's rows
+    int32_t *tile_e = nullptr, *tile_r = nullptr;
+    NfItem *items = nullptr;
+    int32_t nitem = 0, is0 = 0, is1 = 0;     // [is0, is1): the items of FE s's rows
+    uint32_t *split = nullptr;               // bit per row: its sum comes from its item
+    bool stale = false;                      // val does not follow the caches yet
+};
+
+// per-column coefficients of the step, written by the scalar launch
+struct NfCols {
+    double ia[kMaxK], iold[kMaxK];            // v = ia * w, the one before = iold * wold
+    double cq[kMaxK], cv[kMaxK], co[kMaxK];   // w' = cq q + cv w + co wold
+    double chb[kMaxK], cx[kMaxK], ch[kMaxK];  // the h / hbar / x update
+    double beta1[kMaxK];                      // beta of the iteration before
+    int32_t on[kMaxK], upd[kMaxK];            // the column runs; an update goes with the step
+    int32_t due[kMaxK];                       // alpha and the rotations are due
+    int32_t test[kMaxK];                      // the stopping rules are due
+};
+
+struct NfApply {
+    const int32_t *off, *col;
+    const double *val;
+    const int32_t *tile_e, *tile_r;
+    int32_t t0, n0, t1, nt;   // tiles t0 .. t0+n0-1, then t1 .. (nt tiles in all)
+    const double *w;          // p x K
+    double *q;                // p x K: M w
+    double *pa;               // partials [block * K + c]: w'q
+    double *head, *tail;      // [tile * K + c]
+    const int32_t *all_done;
+    double *neg;              // projected, FE s rows: neg[row] = -sum (into w), nothing else
+};
+
+// The scalar step between a product and the step after it.
+struct NfScalars {
+    const double *pa, *pw, *px;
+    int32_t na, nw;           // their lengths (px has pw's)
+    const void *sin;          // LsmrState<double>, K
+    void *sout;               // the same copy in a launch of its own, the other one when folded
+    const NfCols *cin;
+    NfCols *cout;
+    int32_t copy;             // which copy sout is
+    int32_t *all_done;
+};
+// The step's workgroups do the scalar step themselves while each of the
+// partials has at most this many values: up to there two launches an iteration
+// beat three (N = 1e4 to 3.6e4: 20.6 -> 17.5 us an iteration). Past it every
+// workgroup reads too much: with 20000 values (N = 1e7) the step took 22 us,
+// against 7.4 + 5.0 us as two launches.
+constexpr int64_t kNfFold = 2048;
+
+struct NfStep {
+    NfScalars fold;           // cin == nullptr: a launch of its own did it (cols)
+    int64_t p;
+    int64_t row0, rown;       // rows [row0, row0 + rown) are left alone (the eliminated FE)
+    const double *q, *w;
+    double *wold;             // in: the vector before w; out: the next one
+    double *h, *hbar, *x;
+    const NfCols *cols;
+    const NfItem *items;
+    int32_t nitem;
+    const uint32_t *split;
+    const double *head, *tail;
+    double *pw, *px;          // partials ||w'||^2, ||x||^2
+    const int32_t *all_done;
+    unsigned fix_blocks;
+};
+
+// launches (normal.hip); K in {1, 2, 4, 8, 16, 32}
+unsigned nf_apply_blocks(int K, int32_t ntiles);
+void nf_apply(int K, const NfApply &a, unsigned blocks, hipStream_t st);
+void nf_fix_neg(int K, const NfItem *items, int32_t n, const double *head, const double *tail, double *neg,
+                const int32_t *all_done, hipStream_t st);
+void nf_scalars(int K, const NfScalars &s, hipStream_t st);
+void nf_step(int K, const NfStep &s, unsigned blocks, hipStream_t st);
+void nf_init_cols(int K, const void *state, NfCols *cols, hipStream_t st);
+
+// construction (normal.hip), on the handle's stream through its allocator and sort
+struct NfInput {
+    int64_t N = 0;
+    int G = 0, s = 0, t_sec = -1;
+    const int64_t *n = nullptr, *off = nullptr;
+    const int32_t *ref[kMaxG] = {};
+    const double *cache[kMaxG] = {};
+    hipStream_t stream = nullptr;
+};
+// nnz limit for the form to be taken; *fits = 0 leaves m empty
+int nf_build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat &m, int *fits);
+int nf_values(const NfInput &in, NormalMat &m);
+void nf_free(fehip_solver *h, NormalMat &m);
+
+}  // namespace fehip
