@@ -1206,7 +1206,7 @@ struct Plan {
     // v'Mv, ||x||^2 and the step's norm, and the parts of cut rows
     double *nq = nullptr, *nw = nullptr;
     NfCols *ncols = nullptr;
-    void *nstate = nullptr;      // the state's second copy (folded scalar steps)
+    void *nstate = nullptr;      // the state's second copy (folded scalar steps), or the pair kept for the rules
     bool nfold = false;
     int final_copy = 0;          // where the last solve left its state
     double *npa = nullptr, *npx = nullptr, *npw = nullptr, *nhead = nullptr, *ntail = nullptr;
@@ -2859,9 +2859,9 @@ struct Engine {
         P->nblocks = nf_apply_blocks(K, m.ntile);
         P->nfix = (unsigned)std::min(std::max(m.nitem, 1), 1024);
         P->nstep = P->nfix + std::min(grid_for(h->p * K, 4 * kBlock), 1024u);
-        P->nfold = std::max(P->nblocks, P->nstep) * (int64_t)K <= kNfFold;
+        P->nfold = nf_folds(K, P->nblocks, P->nstep);
         CHK(dalloc(h, &P->ncols, 2));
-        CHK(dalloc_bytes(h, &P->nstate, sizeof(LsmrState<double>) * K));
+        CHK(dalloc_bytes(h, &P->nstate, sizeof(LsmrState<double>) * 2 * K));
         CHK(dalloc(h, &P->npa, (size_t)P->nblocks * K));
         CHK(dalloc(h, &P->npx, (size_t)2 * P->nstep * K));
         CHK(dalloc(h, &P->npw, (size_t)2 * P->nstep * K));
@@ -2873,6 +2873,7 @@ struct Engine {
     }
 
     // one LSMR iteration in level space; odd: the current vector is in nw
+    // (iterations 2, 4, .. counted from one)
     static void nf_iteration(fehip_solver *h, Plan *P, bool odd) {
         const NormalMat &m = h->nf;
         double *w = odd ? P->nw : (double *)P->v, *wold = odd ? (double *)P->v : P->nw;
@@ -2908,13 +2909,17 @@ struct Engine {
         }
         nf_apply(K, a, P->nblocks, h->stream);
         // folded, the state, the coefficients and the step's partials alternate
-        // between two copies (the first is current when a solve begins)
+        // between two copies (the first is current when a solve begins); else
+        // h, hbar and x are updated in the steps of iterations 3, 5, ..
         const bool fold = P->nfold;
         const size_t np = (size_t)P->nstep * K;
         NfScalars c{};
         c.pa = P->npa;
         c.pw = P->npw + (fold && !odd ? np : 0);
         c.px = P->npx + (fold && !odd ? np : 0);
+        c.px2 = P->npx + np;
+        c.snap = P->nstate;
+        c.even = odd;
         c.na = (int32_t)P->nblocks;
         c.nw = (int32_t)P->nstep;
         c.sin = fold && odd ? P->nstate : P->state;
@@ -2940,6 +2945,8 @@ struct Engine {
         s.tail = P->ntail;
         s.pw = P->npw + (fold && odd ? np : 0);
         s.px = P->npx + (fold && odd ? np : 0);
+        s.px2 = P->npx + np;
+        s.mode = fold ? kNfFolded : odd ? kNfLight : kNfHeavy;
         s.all_done = P->all_done;
         s.fix_blocks = P->nfix;
         nf_step(K, s, P->nstep, h->stream);

@@ -61,6 +61,10 @@ struct NfCols {
     int32_t on[kMaxK], upd[kMaxK];            // the column runs; an update goes with the step
     int32_t due[kMaxK];                       // alpha and the rotations are due
     int32_t test[kMaxK];                      // the stopping rules are due
+    // updates in pairs: the second one, the column's last iteration is reached,
+    // and x takes the second one back
+    double chb2[kMaxK], cx2[kMaxK], ch2[kMaxK];
+    int32_t upd2[kMaxK], last[kMaxK], undo[kMaxK];
 };
 
 struct NfApply {
@@ -78,24 +82,19 @@ struct NfApply {
 
 // The scalar step between a product and the step after it.
 struct NfScalars {
-    const double *pa, *pw, *px;
-    int32_t na, nw;           // their lengths (px has pw's)
+    const double *pa, *pw, *px, *px2;
+    int32_t na, nw;           // their lengths (px and px2 have pw's)
     const void *sin;          // LsmrState<double>, K
     void *sout;               // the same copy in a launch of its own, the other one when folded
     const NfCols *cin;
     NfCols *cout;
     int32_t copy;             // which copy sout is
     int32_t *all_done;
+    void *snap;               // updates in pairs: the state after the rotations of each, 2 x K
+    int32_t even;             // updates in pairs: 1 in iterations 2, 4, ..
 };
-// The step's workgroups do the scalar step themselves while each of the
-// partials has at most this many values: up to there two launches an iteration
-// beat three (N = 1e4 to 3.6e4: 20.6 -> 17.5 us an iteration). Past it every
-// workgroup reads too much: with 20000 values (N = 1e7) the step took 22 us,
-// against 7.4 + 5.0 us as two launches.
-constexpr int64_t kNfFold = 2048;
-
 struct NfStep {
-    NfScalars fold;           // cin == nullptr: a launch of its own did it (cols)
+    NfScalars fold;           // kNfFolded
     int64_t p;
     int64_t row0, rown;       // rows [row0, row0 + rown) are left alone (the eliminated FE)
     const double *q, *w;
@@ -106,13 +105,17 @@ struct NfStep {
     int32_t nitem;
     const uint32_t *split;
     const double *head, *tail;
-    double *pw, *px;          // partials ||w'||^2, ||x||^2
+    double *pw, *px, *px2;    // partials ||w'||^2, ||x||^2 (after the first and the second update)
     const int32_t *all_done;
     unsigned fix_blocks;
+    int mode;
 };
+// What a step does beside w'.
+enum NfMode { kNfFolded, kNfLight, kNfHeavy };
 
 // launches (normal.hip); K in {1, 2, 4, 8, 16, 32}
 unsigned nf_apply_blocks(int K, int32_t ntiles);
+bool nf_folds(int K, unsigned apply_blocks, unsigned step_blocks);  // the step does the scalar step (kNfFolded)
 void nf_apply(int K, const NfApply &a, unsigned blocks, hipStream_t st);
 void nf_fix_neg(int K, const NfItem *items, int32_t n, const double *head, const double *tail, double *neg,
                 const int32_t *all_done, hipStream_t st);

@@ -474,12 +474,13 @@ __global__ __launch_bounds__(kBlock) void k_nf_fix_neg(const NfItem *items, int3
 
 // one column's entry of NfCols
 struct ColCoef {
-    double ia, iold, cq, cv, co, chb, cx, ch, beta1;
-    int32_t on, upd, due, test;
+    double ia, iold, cq, cv, co, chb, cx, ch, beta1, chb2, cx2, ch2;
+    int32_t on, upd, due, test, upd2, last, undo;
 };
 __device__ __forceinline__ ColCoef load_coef(const NfCols *n, int c) {
-    return {n->ia[c], n->iold[c], n->cq[c], n->cv[c], n->co[c], n->chb[c], n->cx[c], n->ch[c], n->beta1[c],
-            n->on[c], n->upd[c], n->due[c], n->test[c]};
+    return {n->ia[c],   n->iold[c], n->cq[c],  n->cv[c],   n->co[c],   n->chb[c],  n->cx[c],   n->ch[c],  n->beta1[c],
+            n->chb2[c], n->cx2[c],  n->ch2[c], n->on[c],   n->upd[c],  n->due[c],  n->test[c], n->upd2[c], n->last[c],
+            n->undo[c]};
 }
 __device__ __forceinline__ void store_coef(NfCols *n, int c, const ColCoef &f) {
     n->ia[c] = f.ia;
@@ -491,10 +492,41 @@ __device__ __forceinline__ void store_coef(NfCols *n, int c, const ColCoef &f) {
     n->cx[c] = f.cx;
     n->ch[c] = f.ch;
     n->beta1[c] = f.beta1;
+    n->chb2[c] = f.chb2;
+    n->cx2[c] = f.cx2;
+    n->ch2[c] = f.ch2;
     n->on[c] = f.on;
     n->upd[c] = f.upd;
     n->due[c] = f.due;
     n->test[c] = f.test;
+    n->upd2[c] = f.upd2;
+    n->last[c] = f.last;
+    n->undo[c] = f.undo;
+}
+
+// alpha and the rotations of the last iteration, from ||w||^2
+__device__ __forceinline__ void rotate_step(LsmrState<double> &s, ColCoef &f, double wsq, int c, ColOps *ops) {
+    f.iold = f.ia;
+    if (!s.vskip) {
+        const double nw = sqrt(wsq);
+        s.alpha = nw / s.beta;
+        f.ia = nw > 0.0 ? 1.0 / nw : 1.0;
+    }
+    s.inv_alpha = 1.0;
+    fin_rotate<double>(s, c, ops);
+}
+// beta of this iteration from w'Mw, and w'
+__device__ __forceinline__ void beta_step(LsmrState<double> &s, ColCoef &f, double wMw, int c, ColOps *ops) {
+    const double alpha = s.alpha, beta = s.beta;
+    const double vMv = wMw * f.ia * f.ia;
+    const double co = s.iter == 0 ? 0.0 : -(alpha * beta) * f.iold;
+    const double b2 = fma(-alpha, alpha, vMv);  // beta^2 = v'Mv - alpha^2
+    fin_after_db<double>(s, b2 > 0.0 ? b2 : 0.0, MODE_ITER, c, ops);
+    f.beta1 = beta;
+    f.cq = s.vskip ? 0.0 : f.ia;  // beta = 0: v stays (src/utils/lsmr.jl:106)
+    f.cv = s.vskip ? 1.0 : -vMv * f.ia;
+    f.co = s.vskip ? 0.0 : co;
+    f.on = f.due = 1;
 }
 
 // The scalar step of one column, from w'Mw, ||w||^2 and ||x||^2: the stopping
@@ -513,29 +545,86 @@ __device__ __forceinline__ void scalar_step(LsmrState<double> &s, ColCoef &f, do
     f.test = f.on = f.upd = 0;
     if (s.done) return;
     if (f.due) {
-        f.iold = f.ia;
-        if (!s.vskip) {
-            const double nw = sqrt(wsq);
-            s.alpha = nw / s.beta;
-            f.ia = nw > 0.0 ? 1.0 / nw : 1.0;
-        }
-        s.inv_alpha = 1.0;
-        fin_rotate<double>(s, c, ops);
+        rotate_step(s, f, wsq, c, ops);
         f.chb = s.c_hbar;
         f.cx = s.c_x;
         f.ch = s.c_h;
         f.upd = f.test = 1;
     }
-    const double alpha = s.alpha, beta = s.beta;
-    const double vMv = wMw * f.ia * f.ia;
-    const double co = s.iter == 0 ? 0.0 : -(alpha * beta) * f.iold;
-    const double b2 = fma(-alpha, alpha, vMv);  // beta^2 = v'Mv - alpha^2
-    fin_after_db<double>(s, b2 > 0.0 ? b2 : 0.0, MODE_ITER, c, ops);
-    f.beta1 = beta;
-    f.cq = s.vskip ? 0.0 : f.ia;  // beta = 0: v stays (src/utils/lsmr.jl:106)
-    f.cv = s.vskip ? 1.0 : -vMv * f.ia;
-    f.co = s.vskip ? 0.0 : co;
-    f.on = f.due = 1;
+    beta_step(s, f, wMw, c, ops);
+}
+
+// A stopping rule holds whatever ||x|| is (src/utils/lsmr.jl:192-215; ||x||
+// only loosens the two rules on ||r||).
+__device__ __forceinline__ bool stops_anyway(const LsmrState<double> &s) {
+    const double test1 = s.normr / s.normb, test2 = s.normAr / (s.normA * s.normr), test3 = 1.0 / s.condA;
+    return s.iter >= s.maxiter || 1.0 + test3 <= 1.0 || 1.0 + test2 <= 1.0 || 1.0 + test1 <= 1.0 ||
+           test3 <= s.ctol || test2 <= s.atol || test1 <= s.btol;
+}
+
+// The same with the updates of iterations j and j + 1 (j odd) in one step,
+// that of iteration j + 2, which leaves h, hbar and x alone in every other
+// step: 14 vectors read and written in two iterations instead of 20 (32
+// columns, 1.1e6 levels: 198 and 568 us in turn, at 5.6 - 6.4 TB/s, instead of
+// 575 each time; a solve 361 -> 291 ms).  ||x||
+// after both, xsq and xsq2, is known in iteration j + 3 (even): the rules of
+// both are looked at there, on the states a and b kept after their rotations.
+// A column for which a rule holds without ||x|| (nearly always one of these is
+// the first) goes no further (last); where one that needs ||x|| held after j,
+// x takes the update of j + 1 back (undo).  That update is finite then: a
+// rotation breaks down only where alpha = 0, and there stops_anyway held.
+__device__ __forceinline__ void scalar_step_pair(LsmrState<double> &s, ColCoef &f, LsmrState<double> &a,
+                                                 LsmrState<double> &b, bool even, double wMw, double wsq, double xsq,
+                                                 double xsq2, int c, ColOps *ops) {
+    f.on = f.undo = 0;
+    if (s.done) {
+        f.upd = f.upd2 = 0;
+        return;
+    }
+    if (even) {
+        if (f.upd) {
+            fin_after_update<double>(a, xsq, c, ops);
+            bool second = false;
+            if (!a.done && f.upd2) {
+                second = true;
+                fin_after_update<double>(b, xsq2, c, ops);
+            }
+            LsmrState<double> &t = second ? b : a;
+            if (t.done || f.last) {
+                s = t;
+                s.done = 1;
+                f.undo = !second && f.upd2;
+                f.upd = f.upd2 = 0;
+                return;
+            }
+        }
+        f.upd = f.upd2 = 0;
+    }
+    if (f.last) {
+        f.iold = f.ia;  // (its w is the step's wold by now)
+        return;
+    }
+    if (f.due) {
+        rotate_step(s, f, wsq, c, ops);
+        if (even) {
+            f.chb = s.c_hbar;
+            f.cx = s.c_x;
+            f.ch = s.c_h;
+            f.upd = 1;
+            a = s;
+        } else {
+            f.chb2 = s.c_hbar;
+            f.cx2 = s.c_x;
+            f.ch2 = s.c_h;
+            f.upd2 = 1;
+            b = s;
+        }
+        if (stops_anyway(s)) {
+            f.last = 1;
+            return;
+        }
+    }
+    beta_step(s, f, wMw, c, ops);
 }
 
 // Sum of partials [i * K + c] over a thread's share (NT threads, column
@@ -556,100 +645,165 @@ __device__ __forceinline__ double thread_sum(const double *p, int32_t n) {
     return (s0 + s1) + (s2 + s3);
 }
 
-// The scalar step of K columns by NT threads: the column sums of the three
+// The scalar step of K columns by NT threads: the column sums of the
 // partials (lanes, then waves), and thread c < K steps column c in LDS.
-template <int K, int NT>
+template <int K, int NT, bool PAIR>
 struct ScalarMem {
-    double red[3][NT / kWave][K];
-    LsmrState<double> state[K];
+    double red[4][NT / kWave][K];
+    LsmrState<double> state[K], snap[PAIR ? 2 : 1][PAIR ? K : 1];
     ColCoef coef[K];
     ColOps ops;
 };
-template <int K, int NT>
-__device__ __forceinline__ void scalar_block(const NfScalars &p, ScalarMem<K, NT> &m) {
+template <int K, int NT, bool PAIR>
+__device__ __forceinline__ void scalar_block(const NfScalars &p, ScalarMem<K, NT, PAIR> &m) {
     constexpr int W = NT / kWave;
     const int c = threadIdx.x, lane = c & (kWave - 1), wave = c / kWave;
+    const bool even = PAIR && p.even, needx = !PAIR || even;
     if (c < K) {
         m.state[c] = ((const LsmrState<double> *)p.sin)[c];
         m.coef[c] = load_coef(p.cin, c);
     }
+    if constexpr (PAIR)
+        if (even && c >= kWave && c < kWave + 2 * K)
+            m.snap[(c - kWave) / K][(c - kWave) % K] = ((const LsmrState<double> *)p.snap)[c - kWave];
     const double a = column_allreduce<K>(thread_sum<K, NT>(p.pa, p.na));
     const double wsq = column_allreduce<K>(thread_sum<K, NT>(p.pw, p.nw));
-    const double xsq = column_allreduce<K>(thread_sum<K, NT>(p.px, p.nw));
+    const double xsq = needx ? column_allreduce<K>(thread_sum<K, NT>(p.px, p.nw)) : 0.0;
+    const double xsq2 = PAIR && even ? column_allreduce<K>(thread_sum<K, NT>(p.px2, p.nw)) : 0.0;
     if (lane < K) {
         m.red[0][wave][lane] = a;
         m.red[1][wave][lane] = wsq;
         m.red[2][wave][lane] = xsq;
+        m.red[3][wave][lane] = xsq2;
     }
     __syncthreads();
     if (c < K) {
-        double t[3];
-        for (int q = 0; q < 3; q++) {
+        double t[4];
+        for (int q = 0; q < (PAIR ? 4 : 3); q++) {
             double x[4] = {0.0, 0.0, 0.0, 0.0};
             for (int w = 0; w < W; w += 4)
 #pragma unroll
                 for (int u = 0; u < 4; u++) x[u] += m.red[q][w + u][c];
             t[q] = (x[0] + x[1]) + (x[2] + x[3]);
         }
-        scalar_step(m.state[c], m.coef[c], t[0], t[1], t[2], c, &m.ops);
+        if constexpr (PAIR)
+            scalar_step_pair(m.state[c], m.coef[c], m.snap[0][c], m.snap[1][c], even, t[0], t[1], t[2], t[3], c,
+                             &m.ops);
+        else scalar_step(m.state[c], m.coef[c], t[0], t[1], t[2], c, &m.ops);
     }
     __syncthreads();
 }
 // the result of the launch's workgroup 0; *all_done = 1 + the state's copy
-template <int K, int NT>
-__device__ __forceinline__ void scalar_keep(const NfScalars &p, const ScalarMem<K, NT> &m) {
+template <int K, int NT, bool PAIR>
+__device__ __forceinline__ void scalar_keep(const NfScalars &p, const ScalarMem<K, NT, PAIR> &m) {
     const int c = threadIdx.x;
     if (c < K) {
         ((LsmrState<double> *)p.sout)[c] = m.state[c];
         store_coef(p.cout, c, m.coef[c]);
+        if constexpr (PAIR) {
+            const int i = p.even ? 0 : 1;
+            ((LsmrState<double> *)p.snap)[i * K + c] = m.snap[i][c];
+        }
     }
     if (c == 0) {
         int all = 1;
-        for (int q = 0; q < K; q++) all &= m.state[q].done ? 1 : 0;
+        for (int q = 0; q < K; q++) all &= m.state[q].done && !m.coef[q].undo ? 1 : 0;
         if (all) *p.all_done = 1 + p.copy;
     }
 }
 
-// The pending update of hbar, x and h with v = ia w, and w' = cq q + cv w +
-// co wold over wold; ||x||^2 and ||w'||^2.  The first fix_blocks workgroups
-// form w' of the cut rows (split), a workgroup each.
-// FOLD: every workgroup does the scalar step itself first, from the partials of
-// the product and of the step before (a launch less; see kNfFold), and reads
-// and writes alternate copies of the state and of the step's partials.
-template <int K, bool FOLD>
+// The step's workgroups do the scalar step themselves while each of the
+// partials has at most kNfFold values: two launches an iteration then beat
+// three (N = 1e4 to 3.6e4: 20.6 -> 17.5 us an iteration; 24 such panels at once
+// 27.5 -> 24.7 ms). Past it every workgroup reads too much: with 20000 values
+// (N = 1e7) the step took 22 us, against 7.4 + 5.0 us as two launches. And past
+// kNfFoldStep workgroups of the step the updates in pairs, which need the
+// launch, save more than it costs (1.1e6 levels, 1150 workgroups: a solve 23.8
+// folded, 22.4 ms; 2.2e5 levels, 216: 14.4 both).
+constexpr int64_t kNfFold = 2048;
+constexpr unsigned kNfFoldStep = 512;
+
+// w' = cq q + cv w + co wold over wold, ||w'||^2, and by MODE
+//  kNfFolded  the update of hbar, x and h with v = ia w, and ||x||^2.  Every
+//             workgroup does the scalar step itself first, from the partials of
+//             the product and of the step before (a launch less; see kNfFold),
+//             and reads and writes alternate copies of the state and of the
+//             step's partials.
+//  kNfHeavy   two updates, with v = iold wold and v = ia w, and ||x||^2 after each
+//  kNfLight   x takes back its last update in columns that stopped before it
+// The first fix_blocks workgroups have the cut rows (split), one at a time.
+template <int K, int MODE>
 __global__ __launch_bounds__(kBlock) void k_nf_step(NfStep p) {
     if (*p.all_done) return;
+    constexpr bool FOLD = MODE == kNfFolded, HEAVY = MODE == kNfHeavy;
     __shared__ double red[kWavesPerBlock * K];
-    __shared__ ScalarMem<FOLD ? K : 1, kBlock> sm;
+    __shared__ ScalarMem<FOLD ? K : 1, kBlock, false> sm;
     const int tid = threadIdx.x;
     if constexpr (FOLD) {
-        scalar_block<K, kBlock>(p.fold, sm);
-        if (blockIdx.x == 0) scalar_keep<K, kBlock>(p.fold, sm);
+        scalar_block<K, kBlock, false>(p.fold, sm);
+        if (blockIdx.x == 0) scalar_keep<K, kBlock, false>(p.fold, sm);
     }
     auto coef = [&](int c) -> ColCoef {
         if constexpr (FOLD) return sm.coef[c];
         else return load_coef(p.cols, c);
     };
+    // whether x, hbar and h (kNfLight: x and hbar) of the column are touched
+    auto touched = [](const ColCoef &f) { return MODE == kNfLight ? f.undo != 0 : f.upd != 0; };
+    // the updates of one element; w, o = its w and wold; adds to the sums of x^2
+    auto update = [](const ColCoef &f, double &h, double &hb, double &x, double w, double o, double &sx, double &sx2) {
+        if constexpr (MODE == kNfLight) {
+            x -= f.cx2 * hb;
+        } else {
+            hb = hb * f.chb + h;
+            x = x + f.cx * hb;
+            h = h * f.ch + (HEAVY ? o * f.iold : w * f.ia);
+            sx += x * x;
+            if (HEAVY && f.upd2) {
+                hb = hb * f.chb2 + h;
+                x = x + f.cx2 * hb;
+                h = h * f.ch2 + w * f.ia;
+                sx2 += x * x;
+            }
+        }
+    };
     if (blockIdx.x < p.fix_blocks) {
         const int c = tid % K;
         const ColCoef f = coef(c);
-        const bool on = f.on != 0;
-        double acc = 0.0;
+        const bool on = f.on != 0, touch = touched(f);
+        double acc = 0.0, accx = 0.0, accx2 = 0.0;
         for (int32_t i = blockIdx.x; i < p.nitem; i += p.fix_blocks) {
             const NfItem it = p.items[i];
             if (it.row >= p.row0 && it.row < p.row0 + p.rown) continue;
+            const int64_t e = (int64_t)it.row * K + c;
+            double w = 0.0, o = 0.0, h = 0.0, hb = 0.0, x = 0.0;
+            if (tid < K) {
+                w = p.w[e];
+                o = p.wold[e];
+                if (touch) {
+                    if (MODE != kNfLight) h = p.h[e];
+                    hb = p.hbar[e];
+                    x = p.x[e];
+                }
+            }
             const double s = item_sum<K>(it, p.head, p.tail, red);
+            if (tid < K && touch) {
+                update(f, h, hb, x, w, o, accx, accx2);
+                p.x[e] = x;
+                if (MODE != kNfLight) {
+                    p.hbar[e] = hb;
+                    p.h[e] = h;
+                }
+            }
             if (tid < K && on) {
-                const int64_t e = (int64_t)it.row * K + c;
-                const double w = p.w[e];
-                const double n = f.cq * (w + s) + f.cv * w + f.co * p.wold[e];
+                const double n = f.cq * (w + s) + f.cv * w + f.co * o;
                 p.wold[e] = n;
                 acc += n * n;
             }
         }
         if (tid < K) {
             p.pw[(int64_t)blockIdx.x * K + tid] = acc;
-            p.px[(int64_t)blockIdx.x * K + tid] = 0.0;
+            if (MODE != kNfLight) p.px[(int64_t)blockIdx.x * K + tid] = accx;
+            if (HEAVY) p.px2[(int64_t)blockIdx.x * K + tid] = accx2;
         }
         return;
     }
@@ -657,43 +811,36 @@ __global__ __launch_bounds__(kBlock) void k_nf_step(NfStep p) {
     constexpr int V = K == 1 ? 1 : 2, KV = K / V, U = 4 / V;
     using Vec = VecC<double, V>;
     const int c0 = tid % KV * V;
-    double ia[V], cq[V], cv[V], co[V], chb[V], cx[V], ch[V];
-    bool on[V], upd[V], any = false, anyu = false;
+    ColCoef f[V];
+    bool on[V], touch[V], any = false, anyu = false;
 #pragma unroll
     for (int v = 0; v < V; v++) {
-        const ColCoef f = coef(c0 + v);
-        on[v] = f.on != 0;
-        upd[v] = f.upd != 0;
+        f[v] = coef(c0 + v);
+        on[v] = f[v].on != 0;
+        touch[v] = touched(f[v]);
         any |= on[v];
-        anyu |= upd[v];
-        ia[v] = f.ia;
-        cq[v] = f.cq;
-        cv[v] = f.cv;
-        co[v] = f.co;
-        chb[v] = f.chb;
-        cx[v] = f.cx;
-        ch[v] = f.ch;
+        anyu |= touch[v];
     }
-    double acc[V] = {}, accx[V] = {};
-    if (any) {
+    double acc[V] = {}, accx[V] = {}, accx2[V] = {};
+    if (any || anyu) {
         const int64_t n = (p.p - p.rown) * KV, skip0 = p.row0 * KV, skipn = p.rown * KV;
         const int64_t stride = (int64_t)(gridDim.x - p.fix_blocks) * kBlock;
         for (int64_t b = (int64_t)(blockIdx.x - p.fix_blocks) * kBlock + tid; b < n; b += U * stride) {
             uint32_t ee[U];
             Vec q[U], w[U], o[U], h[U], hb[U], x[U];
-            bool in[U], sp[U];
+            bool in[U];
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 in[u] = b + u * stride < n;
                 const int64_t e = in[u] ? b + u * stride : b;
                 const uint32_t at = (uint32_t)(e < skip0 ? e : e + skipn), r = at / KV;
                 ee[u] = at * V;
-                sp[u] = (p.split[r >> 5] >> (r & 31)) & 1;
+                if ((p.split[r >> 5] >> (r & 31)) & 1) in[u] = false;
                 q[u] = ldv<V>(p.q, ee[u]);
                 w[u] = ldv<V>(p.w, ee[u]);
                 o[u] = ldv<V>((const double *)p.wold, ee[u]);
                 if (anyu) {
-                    h[u] = ldv<V>((const double *)p.h, ee[u]);
+                    if (MODE != kNfLight) h[u] = ldv<V>((const double *)p.h, ee[u]);
                     hb[u] = ldv<V>((const double *)p.hbar, ee[u]);
                     x[u] = ldv<V>((const double *)p.x, ee[u]);
                 }
@@ -703,22 +850,20 @@ __global__ __launch_bounds__(kBlock) void k_nf_step(NfStep p) {
                 if (!in[u]) continue;
                 if (anyu) {
 #pragma unroll
-                    for (int v = 0; v < V; v++) {
-                        if (!upd[v]) continue;
-                        hb[u].v[v] = hb[u].v[v] * chb[v] + h[u].v[v];
-                        x[u].v[v] = x[u].v[v] + cx[v] * hb[u].v[v];
-                        h[u].v[v] = h[u].v[v] * ch[v] + w[u].v[v] * ia[v];
-                        accx[v] += x[u].v[v] * x[u].v[v];
-                    }
-                    stv<V>(p.hbar, ee[u], hb[u]);
+                    for (int v = 0; v < V; v++)
+                        if (touch[v])
+                            update(f[v], h[u].v[v], hb[u].v[v], x[u].v[v], w[u].v[v], o[u].v[v], accx[v], accx2[v]);
                     stv<V>(p.x, ee[u], x[u]);
-                    stv<V>(p.h, ee[u], h[u]);
+                    if (MODE != kNfLight) {
+                        stv<V>(p.hbar, ee[u], hb[u]);
+                        stv<V>(p.h, ee[u], h[u]);
+                    }
                 }
-                if (sp[u]) continue;
+                if (!any) continue;
 #pragma unroll
                 for (int v = 0; v < V; v++) {
                     if (!on[v]) continue;
-                    o[u].v[v] = cq[v] * q[u].v[v] + cv[v] * w[u].v[v] + co[v] * o[u].v[v];
+                    o[u].v[v] = f[v].cq * q[u].v[v] + f[v].cv * w[u].v[v] + f[v].co * o[u].v[v];
                     acc[v] += o[u].v[v] * o[u].v[v];
                 }
                 stv<V>(p.wold, ee[u], o[u]);
@@ -729,8 +874,14 @@ __global__ __launch_bounds__(kBlock) void k_nf_step(NfStep p) {
     for (int v = 0; v < V; v++) {
         const double s = block_column_sum<KV>(acc[v], red);
         if (tid < KV) p.pw[(int64_t)blockIdx.x * K + tid * V + v] = s;
-        const double sx = block_column_sum<KV>(accx[v], red);
-        if (tid < KV) p.px[(int64_t)blockIdx.x * K + tid * V + v] = sx;
+        if (MODE != kNfLight) {
+            const double sx = block_column_sum<KV>(accx[v], red);
+            if (tid < KV) p.px[(int64_t)blockIdx.x * K + tid * V + v] = sx;
+        }
+        if (HEAVY) {
+            const double sx = block_column_sum<KV>(accx2[v], red);
+            if (tid < KV) p.px2[(int64_t)blockIdx.x * K + tid * V + v] = sx;
+        }
     }
 }
 
@@ -738,9 +889,9 @@ __global__ __launch_bounds__(kBlock) void k_nf_step(NfStep p) {
 template <int K>
 __global__ __launch_bounds__(kFinBlock) void k_nf_scalars(NfScalars p) {
     if (*p.all_done) return;
-    __shared__ ScalarMem<K, kFinBlock> sm;
-    scalar_block<K, kFinBlock>(p, sm);
-    scalar_keep<K, kFinBlock>(p, sm);
+    __shared__ ScalarMem<K, kFinBlock, true> sm;
+    scalar_block<K, kFinBlock, true>(p, sm);
+    scalar_keep<K, kFinBlock, true>(p, sm);
 }
 
 __global__ void k_nf_init_cols(const LsmrState<double> *st, int K, NfCols *cols) {
@@ -753,6 +904,8 @@ __global__ void k_nf_init_cols(const LsmrState<double> *st, int K, NfCols *cols)
     cols->beta1[c] = 0.0;
     cols->on[c] = c < K && !st[c].done ? 1 : 0;
     cols->upd[c] = cols->due[c] = cols->test[c] = 0;
+    cols->chb2[c] = cols->cx2[c] = cols->ch2[c] = 0.0;
+    cols->upd2[c] = cols->last[c] = cols->undo[c] = 0;
 }
 
 template <int K>
@@ -817,6 +970,9 @@ void nf_fix_neg(int K, const NfItem *items, int32_t n, const double *head, const
     });
 }
 
+bool nf_folds(int K, unsigned apply_blocks, unsigned step_blocks) {
+    return (int64_t)std::max(apply_blocks, step_blocks) * K <= kNfFold && step_blocks <= kNfFoldStep;
+}
 void nf_scalars(int K, const NfScalars &a, hipStream_t st) {
     for_width(K, [&](auto k) {
         hipLaunchKernelGGL((k_nf_scalars<decltype(k)::value>), dim3(1), dim3(kFinBlock), 0, st, a);
@@ -826,8 +982,10 @@ void nf_scalars(int K, const NfScalars &a, hipStream_t st) {
 void nf_step(int K, const NfStep &s, unsigned blocks, hipStream_t st) {
     for_width(K, [&](auto k) {
         constexpr int W = decltype(k)::value;
-        if (s.fold.cin) hipLaunchKernelGGL((k_nf_step<W, true>), dim3(blocks), dim3(kBlock), 0, st, s);
-        else hipLaunchKernelGGL((k_nf_step<W, false>), dim3(blocks), dim3(kBlock), 0, st, s);
+        auto kernel = s.mode == kNfFolded  ? k_nf_step<W, kNfFolded>
+                      : s.mode == kNfHeavy ? k_nf_step<W, kNfHeavy>
+                                           : k_nf_step<W, kNfLight>;
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), 0, st, s);
     });
 }
 
