@@ -191,6 +191,9 @@ struct fehip_solver {
     int32_t *cc_nodes = nullptr;  // p
     int32_t *cc_start = nullptr;  // p + 2
     uint32_t *cc_ncomp = nullptr; // 1
+    int32_t *cc_big = nullptr;    // components of more than kRescaleBig levels
+    int32_t cc_nbig = 0;
+    double *cc_part = nullptr;    // their partial sums and counts
     // level-space form of the FP64 iteration (normal.h), built at the first
     // solve: 0 not looked at, 1 built, -1 not taken (FEHIP_NORMAL=0, or too
     // many entries)
@@ -3649,6 +3652,12 @@ static int ensure_components(fehip_solver *h) {
         prm.node0[j] = h->off[idx[j]];
     }
     prm.nu = (int32_t)idx.size();
+    if (h->N >= kCcRounds)
+        for (int64_t stride : {16, 16, 16, 4, 4, 4}) {
+            hipLaunchKernelGGL(k_cc_round, dim3(grid_for((h->N + stride - 1) / stride, kBlock)), dim3(kBlock), 0,
+                               h->stream, prm, h->N, stride, parent);
+            hipLaunchKernelGGL(k_cc_flatten, dim3(grid_for(p, kBlock)), dim3(kBlock), 0, h->stream, parent, p);
+        }
     hipLaunchKernelGGL(k_cc_hook, dim3(grid_for(h->N, kBlock)), dim3(kBlock), 0, h->stream, prm, h->N, parent,
                        seen);
     hipLaunchKernelGGL(k_cc_roots, dim3(grid_for(p, kBlock)), dim3(kBlock), 0, h->stream, parent,
@@ -3663,7 +3672,19 @@ static int ensure_components(fehip_solver *h) {
                        (const int32_t *)skeys, p, h->cc_start);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(h->cc_ncomp, rid + p, sizeof(uint32_t), hipMemcpyDeviceToDevice, h->stream));
+    // components too large for one workgroup
+    uint32_t *bcount = nullptr, nbig = 0;
+    CHK(dalloc(h, &bcount, 1));
+    CHK(dalloc(h, &h->cc_big, p / kRescaleBig + 1));
+    hipLaunchKernelGGL(k_fill<uint32_t>, dim3(1), dim3(64), 0, h->stream, bcount, (int64_t)1, 0u);
+    hipLaunchKernelGGL(k_cc_big, dim3(grid_for(p, kBlock)), dim3(kBlock), 0, h->stream,
+                       (const int32_t *)h->cc_start, (const uint32_t *)h->cc_ncomp, p, h->cc_big, bcount);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(&nbig, bcount, sizeof(nbig), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
+    h->cc_nbig = (int32_t)nbig;
+    if (nbig) CHK(dalloc(h, &h->cc_part, (size_t)nbig * kRescaleBlocks * 2 * kMaxG));
+    dfree(h, bcount);
     dfree(h, parent);
     dfree(h, seen);
     dfree(h, flag);
@@ -3690,6 +3711,14 @@ static int normalize_dev(fehip_solver *h, double *dc) {
     const unsigned grid = (unsigned)std::min<int64_t>(h->p, 1024);
     hipLaunchKernelGGL(k_rescale, dim3(grid), dim3(kBlock), 0, h->stream, prm, (const int32_t *)h->cc_nodes,
                        (const int32_t *)h->cc_start, (const uint32_t *)h->cc_ncomp, dc);
+    for (int32_t b0 = 0; b0 < h->cc_nbig; b0 += 65535) {
+        const dim3 gr(kRescaleBlocks, (unsigned)std::min(h->cc_nbig - b0, 65535));
+        double *part = h->cc_part + (size_t)b0 * kRescaleBlocks * 2 * kMaxG;
+        hipLaunchKernelGGL(k_rescale_part, gr, dim3(kBlock), 0, h->stream, prm, (const int32_t *)h->cc_nodes,
+                           (const int32_t *)h->cc_start, (const int32_t *)h->cc_big + b0, (const double *)dc, part);
+        hipLaunchKernelGGL(k_rescale_apply, gr, dim3(kBlock), 0, h->stream, prm, (const int32_t *)h->cc_nodes,
+                           (const int32_t *)h->cc_start, (const int32_t *)h->cc_big + b0, (const double *)part, dc);
+    }
     HIPCHK(hipGetLastError());
     return 0;
 }
