@@ -6,9 +6,10 @@
 // sorted with their observation index; a level starts wherever the sorted key
 // changes, a scan numbers the levels, and the numbers are scattered back to
 // the observations.  Levels are therefore numbered in ascending key order.
-// Several columns: each is numbered alone, then the numbers are combined as
-// prev * n_next + next (lexicographic order) and the combination is numbered
-// again.
+// Several columns: where the widths of their ranges add up to at most 64 bits,
+// the offsets share one word and are numbered as one key.  Otherwise each is
+// numbered alone, then the numbers are combined as prev * n_next + next
+// (lexicographic order) and the combination is numbered again.
 #pragma once
 
 #include "fehip_common.h"
