@@ -119,6 +119,24 @@ def kernel_bytes(N, n, kinds, K, s, factored, weighted, plan):
     return out
 
 
+def level_bytes(panel, K):
+    """Algorithmic HBM bytes per launch of the level-space iteration: M = A'A
+    has two entries per distinct pair of levels (a column number and a value),
+    its diagonal is 1.  The step writes the next vector from three and updates
+    h, hbar and x for two iterations in every other launch (the mean; a small
+    problem, whose step does the scalar step too, updates them in each)."""
+    G, p = len(panel.n), sum(int(k) for k in panel.n)
+    nnz = 0
+    for a in range(G):
+        for b in range(a + 1, G):
+            key = np.asarray(panel.refs[a], np.int64) * (int(panel.n[b]) + 1) + np.asarray(panel.refs[b], np.int64)
+            key.sort()
+            nnz += 2 * (1 + int(np.count_nonzero(key[1:] != key[:-1])))
+    out = {"k_nf_apply": 12 * nnz + 4 * (p + 1) + 16 * K * p, "k_nf_step": 7 * 8 * K * p}
+    out["pair"] = out["k_nf_apply"]  # D*v and D'u in one product
+    return out
+
+
 def cpu_model():
     try:
         for line in open("/proc/cpuinfo"):
@@ -173,7 +191,8 @@ KERNEL_NAMES = ["k_fused", "k_fin_db", "k_dtx_csr", "k_dtx_dense", "k_dtx_fixup"
 def kernel_report(feM, panel, K, precision, name, form_key=None):
     """Per-kernel HIP-event times of one iteration (fehip_time_kernels on the
     handle's stream), the dominant kernel's roofline entry, and the survey's
-    pair-formula bytes over the iteration's D*x + D'u launches."""
+    pair-formula bytes over the iteration's D*x + D'u launches (in level space:
+    the product's own bytes over its time)."""
     import ctypes as C
 
     from fixedeffects_rocm._lib import check, lib
@@ -189,15 +208,21 @@ def kernel_report(feM, panel, K, precision, name, form_key=None):
     s = 4 if fp32 else 8
     kb = kernel_bytes(panel.N, list(panel.n), kinds, K, s, factored, panel.weights is not None, plan)
     kt = {nm: float(m) for nm, m in zip(KERNEL_NAMES, ms)}
-    dom = max(["k_fused", "k_dtx_csr", "k_dtx_dense", "k_dtx_fixup", "k_update"], key=lambda q: kt[q])
+    form = "pieces" if plan["pieces"] else "csr"
+    if kt["k_fin_dtx"] == 0.0:  # the iteration in level space: three launches, FP64 in both modes
+        form = "level"
+        kb = level_bytes(panel, K)
+        kt = {nm: kt[q] for nm, q in (("k_nf_apply", "k_fused"), ("k_nf_scalars", "k_fin_db"),
+                                      ("k_nf_step", "k_update"), ("event_pair", "event_pair"))}
+    dom = max([q for q in ["k_fused", "k_dtx_csr", "k_dtx_dense", "k_dtx_fixup", "k_update", "k_nf_apply",
+               "k_nf_step"] if q in kt], key=lambda q: kt[q])
     # the launch's duration: its event interval less the interval of an empty
     # event pair recorded the same way on the same stream (the timing's own
     # cost, which every interval includes)
     ovh = kt["event_pair"] if 0.0 < kt["event_pair"] < 0.5 * kt[dom] else 0.0
     dur_ms = kt[dom] - ovh
     achieved = kb[dom] / (dur_ms * 1e-3) / 1e9
-    pair_ms = sum(kt[q] for q in KERNEL_NAMES[:6])
-    form = "pieces" if plan["pieces"] else "csr"
+    pair_ms = kt["k_nf_apply"] if form == "level" else sum(kt[q] for q in KERNEL_NAMES[:6])
     traffic, src = PMC_TRAFFIC.get((name, precision, K, form), ({}, None))
     roof = {"bound": "hbm", "kernel": dom, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic.get(dom), "traffic_source": src if traffic else None,
@@ -476,6 +501,7 @@ def main():
         "config": {"workload": name, "N": N, "levels": [int(k) for k in panel.n], "K": K, "tol": args.tol,
                    "weights": "LogNormal(0,0.5)", "precision": args.precision,
                    "mode": ("plain LSMR, reference start" if args.precision == "fp64"
+                            else "FP64 iterations in level space" if rep["form"] == "level"
                             else "FP32-stream LSMR phase, then FP64 LSMR iterations from its solution")
                    + ("" if args.algorithm == "lsmr" else "; projected LSMR (FE of most levels eliminated)"),
                    "algorithm": args.algorithm},

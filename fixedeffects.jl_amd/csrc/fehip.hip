@@ -2614,17 +2614,8 @@ struct Engine {
         hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(pK, kBlock)), dim3(kBlock), 0, h->stream, (T *)P->x, pK, (T)0);
         hipLaunchKernelGGL((k_lsmr_setup<Tr>), dim3(1), dim3(64), 0, h->stream, (LsmrState<Tr> *)P->state, K, K, 0.0,
                            0.0, 0.0, (int64_t)1 << 40, P->all_done);
-        hipLaunchKernelGGL(k_set_ops, dim3(1), dim3(64), 0, h->stream, P->ops_once, -1.0, 1.0, K, K);
-        db(h, P, MODE_INIT, P->ops_once, (const T *)P->x, (T *)P->u, nullptr);
-        fin_db(h, P, MODE_INIT, nullptr);
-        dtx(h, P, MODE_INIT, P->ops_dtx, (const T *)P->u, (T *)P->v, nullptr);
-        fin_dtx(h, P, MODE_INIT, nullptr);
-        hipLaunchKernelGGL((k_init_vectors<T, Tr, K>), dim3(P->upd_blocks), dim3(kBlock), 0, h->stream, pK, (T *)P->v,
-                           (T *)P->hh, (T *)P->hbar, (const void *)P->state, (const T *)h->scale_all[pidx<T>()],
-                           (T *)P->vt);
-        if (ut_now(h, P) && h->sqrtw_T[pidx<T>()])
-            hipLaunchKernelGGL(k_scale_rows<T>, dim3(grid_for(NK, kBlock)), dim3(kBlock), 0, h->stream, (T *)P->u,
-                               (const T *)h->sqrtw_T[pidx<T>()], h->N, K);
+        CHK(lsmr_init(h, P, K));
+        CHK(lsmr_vectors(h, P, false));
         HIPCHK(hipGetLastError());
         hipEvent_t ev[10];
         for (auto &e : ev) HIPCHK(hipEventCreate(&e));
@@ -2858,6 +2849,34 @@ struct Engine {
         update(h, P);
     }
 
+    // u = b - A x ; beta = ||u||  (:63-65) ; v = A'u ; alpha = ||v|| and the
+    // scalar set-up  (:66-98)
+    static int lsmr_init(fehip_solver *h, Plan *P, int Kreal) {
+        hipLaunchKernelGGL(k_set_ops, dim3(1), dim3(64), 0, h->stream, P->ops_once, -1.0, 1.0, K, Kreal);
+        db(h, P, MODE_INIT, P->ops_once, (const T *)P->x, (T *)P->u, nullptr);
+        fin_db(h, P, MODE_INIT, nullptr);
+        dtx(h, P, MODE_INIT, P->ops_dtx, (const T *)P->u, (T *)P->v, nullptr);
+        fin_dtx(h, P, MODE_INIT, nullptr);
+        return 0;
+    }
+
+    // v normalized, h = v, hbar = 0, and what the form of the iteration keeps beside
+    static int lsmr_vectors(fehip_solver *h, Plan *P, bool nf) {
+        hipLaunchKernelGGL((k_init_vectors<T, Tr, K>), dim3(P->upd_blocks), dim3(kBlock), 0, h->stream, h->p * K,
+                           (T *)P->v, (T *)P->hh, (T *)P->hbar, (const void *)P->state,
+                           (const T *)h->scale_all[pidx<T>()], nf ? (T *)nullptr : (T *)P->vt);
+        if (nf) {
+            hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream, P->nw,
+                               h->p * K, 0.0);
+            nf_init_cols(K, P->state, P->ncols, h->stream);
+        } else if (ut_now(h, P) && h->sqrtw_T[pidx<T>()])
+            // the factored iteration with K < 8 keeps u as sqrt(w) .* u (not
+            // the piece form)
+            hipLaunchKernelGGL(k_scale_rows<T>, dim3(grid_for(h->N * K, kBlock)), dim3(kBlock), 0, h->stream,
+                               (T *)P->u, (const T *)h->sqrtw_T[pidx<T>()], h->N, K);
+        return 0;
+    }
+
     // the level-space iteration (normal.h) is in use: FP64 on a handle that has M
     static bool use_nf(const fehip_solver *h, const Plan *P) { return sizeof(T) == 8 && h->nf_state == 1 && P->nq; }
 
@@ -2883,7 +2902,12 @@ struct Engine {
 
     // one LSMR iteration in level space; odd: the current vector is in nw
     // (iterations 2, 4, .. counted from one)
-    static void nf_iteration(fehip_solver *h, Plan *P, bool odd) {
+    // mark(0..3): before each launch and after the last
+    struct NoMark {
+        void operator()(int) const {}
+    };
+    template <typename Mark = NoMark>
+    static void nf_iteration(fehip_solver *h, Plan *P, bool odd, Mark mark = Mark()) {
         const NormalMat &m = h->nf;
         double *w = odd ? P->nw : (double *)P->v, *wold = odd ? (double *)P->v : P->nw;
         NfApply a{};
@@ -2916,7 +2940,9 @@ struct Engine {
             s.row0 = h->off[h->s];
             s.rown = h->n[h->s];
         }
+        mark(0);
         nf_apply(K, a, P->nblocks, h->stream);
+        mark(1);
         // folded, the state, the coefficients and the step's partials alternate
         // between two copies (the first is current when a solve begins); else
         // h, hbar and x are updated in the steps of iterations 3, 5, ..
@@ -2939,6 +2965,7 @@ struct Engine {
         c.all_done = P->all_done;
         if (fold) s.fold = c;
         else nf_scalars(K, c, h->stream);
+        mark(2);
         s.p = h->p;
         s.q = P->nq;
         s.w = w;
@@ -2959,6 +2986,43 @@ struct Engine {
         s.all_done = P->all_done;
         s.fix_blocks = P->nfix;
         nf_step(K, s, P->nstep, h->stream);
+        mark(3);
+    }
+
+    // fehip_time_kernels where the level-space iteration is in use
+    static int time_level(fehip_solver *h, int reps, double *out_ms) {
+        Plan *P = nullptr;
+        CHK((get_plan_for<T, Acc, K>(h, &P)));
+        CHK(nf_plan(h, P));
+        const int64_t NK = h->N * K, pK = h->p * K;
+        hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(NK, kBlock)), dim3(kBlock), 0, h->stream, (T *)P->u, NK, (T)1);
+        hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(pK, kBlock)), dim3(kBlock), 0, h->stream, (T *)P->x, pK, (T)0);
+        hipLaunchKernelGGL((k_lsmr_setup<Tr>), dim3(1), dim3(64), 0, h->stream, (LsmrState<Tr> *)P->state, K, K, 0.0,
+                           0.0, 0.0, (int64_t)1 << 40, P->all_done);
+        CHK(lsmr_init(h, P, K));
+        CHK(lsmr_vectors(h, P, true));
+        HIPCHK(hipGetLastError());
+        hipEvent_t ev[5];
+        for (auto &e : ev) HIPCHK(hipEventCreate(&e));
+        double acc[4] = {0, 0, 0, 0};
+        for (int r = -2; r < (reps + 1) / 2 * 2; r++) {
+            nf_iteration(h, P, r & 1, [&](int q) { (void)hipEventRecord(ev[q], h->stream); });
+            HIPCHK(hipEventRecord(ev[4], h->stream));
+            HIPCHK(hipEventSynchronize(ev[4]));
+            for (int q = 0; r >= 0 && q < 4; q++) {
+                float ms = 0.f;
+                HIPCHK(hipEventElapsedTime(&ms, ev[q], ev[q + 1]));
+                acc[q] += ms;
+            }
+        }
+        for (auto &e : ev) (void)hipEventDestroy(e);
+        int32_t stopped = 0;
+        HIPCHK(hipMemcpy(&stopped, P->all_done, sizeof(int32_t), hipMemcpyDeviceToHost));
+        if (stopped) return fail(FEHIP_EHIP, "kernel timing: the filler LSMR stopped early");
+        for (int q = 0; q < 8; q++) out_ms[q] = 0.0;
+        const int slot[4] = {0, 1, 6, 7};
+        for (int q = 0; q < 4; q++) out_ms[slot[q]] = acc[q] / ((reps + 1) / 2 * 2);
+        return 0;
     }
 
     static int ensure_graph(fehip_solver *h, Plan *P) {
@@ -3034,26 +3098,9 @@ struct Engine {
             dtx_fixup(h, P, MODE_INIT, P->ops_dtx, (T *)P->v, nullptr, false, true);
             fin_dtx(h, P, MODE_INIT, nullptr, true);
         } else {
-            // u = b - A x ; beta = ||u||  (:63-65)
-            hipLaunchKernelGGL(k_set_ops, dim3(1), dim3(64), 0, h->stream, P->ops_once, -1.0, 1.0, K, Kreal);
-            db(h, P, MODE_INIT, P->ops_once, (const T *)P->x, (T *)P->u, nullptr);
-            fin_db(h, P, MODE_INIT, nullptr);
-            // v = A'u ; alpha = ||v|| and the scalar set-up  (:66-98)
-            dtx(h, P, MODE_INIT, P->ops_dtx, (const T *)P->u, (T *)P->v, nullptr);
-            fin_dtx(h, P, MODE_INIT, nullptr);
+            CHK(lsmr_init(h, P, Kreal));
         }
-        hipLaunchKernelGGL((k_init_vectors<T, Tr, K>), dim3(P->upd_blocks), dim3(kBlock), 0, h->stream, h->p * K,
-                           (T *)P->v, (T *)P->hh, (T *)P->hbar, (const void *)P->state,
-                           (const T *)h->scale_all[pidx<T>()], nf ? (T *)nullptr : (T *)P->vt);
-        if (nf) {
-            hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream, P->nw,
-                               h->p * K, 0.0);
-            nf_init_cols(K, P->state, P->ncols, h->stream);
-        } else if (ut_now(h, P) && h->sqrtw_T[pidx<T>()])
-            // the factored iteration with K < 8 keeps u as sqrt(w) .* u (not
-            // the piece form)
-            hipLaunchKernelGGL(k_scale_rows<T>, dim3(grid_for(h->N * K, kBlock)), dim3(kBlock), 0, h->stream,
-                               (T *)P->u, (const T *)h->sqrtw_T[pidx<T>()], h->N, K);
+        CHK(lsmr_vectors(h, P, nf));
         HIPCHK(hipGetLastError());
         CHK(ensure_graph(h, P));
         // Two replays in flight: while the host waits on replay i's copy of
@@ -4478,6 +4525,12 @@ int fehip_time_kernels(fehip_t *h, int32_t K, int32_t reps, double *out_ms) {
     g_err.clear();
     if (!h || !out_ms) return fail(FEHIP_EARG, "bad arguments");
     if (K < 1 || K > kMaxK || reps < 1) return fail(FEHIP_EARG, "K must be in 1..32 and reps >= 1");
+    if (h->precision != FEHIP_FP32 && h->G > 1) {
+        CHK(ensure_normal(h));
+        if (h->nf_state == 1)
+            return for_K<double, double, double>(padded_K(K),
+                                                 [&](auto e) { return decltype(e)::time_level(h, reps, out_ms); });
+    }
     return dispatch(h->precision, padded_K(K), [&](auto e) { return decltype(e)::time_kernels(h, reps, out_ms); });
 }
 

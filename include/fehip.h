@@ -315,7 +315,15 @@ int fehip_plan_info(fehip_t *h, int32_t K, int32_t fp32_storage, int64_t *out);
  *   out_ms[7] two events recorded back to back with no launch between
  *             them: the timing's own overhead, included in every slot above
  *             (the ||x|| and stopping-rule step runs inside the next
- *             iteration's beta finalize, out_ms[1]) */
+ *             iteration's beta finalize, out_ms[1])
+ * Where the FP64 iteration runs in level space (FEHIP_FP64 and FEHIP_MIXED
+ * handles whose normal matrix is built), its launches instead:
+ *   out_ms[0] q = M v, M the normal matrix over the levels, and v'q
+ *   out_ms[1] the scalar step: stopping rules, rotations, beta (about the
+ *             empty pair where the vector step's workgroups do it)
+ *   out_ms[6] the vector step: the next v, and h, hbar and x; the mean over
+ *             an even number of iterations
+ * and 0 in out_ms[2..5]. */
 int fehip_time_kernels(fehip_t *h, int32_t K, int32_t reps, double *out_ms);
 
 /* Schedule of the LSMR launches (no reference counterpart; the reference's
