@@ -1195,9 +1195,10 @@ struct Plan {
     int32_t *all_done = nullptr;
     void *u = nullptr, *r = nullptr, *x = nullptr, *v = nullptr, *hh = nullptr, *hbar = nullptr;
     double *dY = nullptr;  // staging for host columns (N x K doubles)
-    hipGraphExec_t graph = nullptr;
-    int graph_iters = 0;
-    bool graph_fwl = false;
+    // captured iterations: over the observations, in level space
+    hipGraphExec_t graph[2] = {};
+    int graph_iters[2] = {};
+    bool graph_fwl[2] = {};
     // projected iteration: FE s items (crossing segments, into zs from level
     // 0), the other FEs' items, zs = the FE s correction (n_s x K)
     FixItem *items_s = nullptr, *items_o = nullptr;
@@ -1214,6 +1215,7 @@ struct Plan {
     // current and the previous one, per-column coefficients, partials of
     // v'Mv, ||x||^2 and the step's norm, and the parts of cut rows
     double *nq = nullptr, *nw = nullptr;
+    double *nx0 = nullptr;       // the solve's first x, for a start over
     NfCols *ncols = nullptr;
     void *nstate = nullptr;      // the state's second copy (folded scalar steps), or the pair kept for the rules
     bool nfold = false;
@@ -1707,22 +1709,24 @@ static int get_plan_for(fehip_solver *h, Plan **out) {
 }
 
 static void destroy_plan(fehip_solver *h, Plan *P) {
-    if (P->graph) (void)hipGraphExecDestroy(P->graph);
+    for (hipGraphExec_t g : P->graph)
+        if (g) (void)hipGraphExecDestroy(g);
     void *ptrs[] = {P->items, P->tileA, P->tileB, P->dpart, P->part_db, P->part_seg, P->part_fix, P->part_upd,
                     P->part_fused, P->wsum, P->sdirect, P->vt, P->state, P->ops_db, P->ops_dtx, P->ops_once, P->all_done, P->u, P->r, P->x,
                     P->v, P->hh, P->hbar, P->dY, P->tstart, P->items_s, P->items_o, P->items_sd, P->items_c,
                     P->zs, P->ops_one, P->ops_neg, P->ops_sub, P->items_d, P->nq, P->nw, P->ncols, P->npa, P->npx,
-                    P->npw, P->nhead, P->ntail, P->nstate};
+                    P->npw, P->nhead, P->ntail, P->nstate, P->nx0};
     for (void *q : ptrs) dfree(h, q);
     destroy_pieces(h, P->pc);
     delete P;
 }
 
 static void drop_graphs(fehip_solver *h) {
-    for (auto &kv : h->plans) {
-        if (kv.second->graph) (void)hipGraphExecDestroy(kv.second->graph);
-        kv.second->graph = nullptr;
-    }
+    for (auto &kv : h->plans)
+        for (hipGraphExec_t &g : kv.second->graph) {
+            if (g) (void)hipGraphExecDestroy(g);
+            g = nullptr;
+        }
 }
 
 static void destroy_all_plans(fehip_solver *h) {
@@ -2896,6 +2900,7 @@ struct Engine {
         CHK(dalloc(h, &P->nhead, (size_t)m.ntile * K));
         CHK(dalloc(h, &P->ntail, (size_t)m.ntile * K));
         CHK(dalloc(h, &P->nw, (size_t)h->p * K));
+        CHK(dalloc(h, &P->nx0, (size_t)h->p * K));
         CHK(dalloc(h, &P->nq, (size_t)h->p * K));
         return 0;
     }
@@ -3025,22 +3030,22 @@ struct Engine {
         return 0;
     }
 
-    static int ensure_graph(fehip_solver *h, Plan *P) {
-        const bool nf = use_nf(h, P);
+    static int ensure_graph(fehip_solver *h, Plan *P, bool nf) {
         // (the level-space iterations alternate two vectors: an even number per graph)
         const int M = nf ? (h->poll_iters + 1) / 2 * 2 : h->poll_iters;
-        if (P->graph && P->graph_iters == M && P->graph_fwl == h->fwl_now) return 0;
+        hipGraphExec_t &graph = P->graph[nf];
+        if (graph && P->graph_iters[nf] == M && P->graph_fwl[nf] == h->fwl_now) return 0;
         // the split fix-up's second stream exists only on handles whose graph
         // uses it: every stream of the process shares a few hardware queues,
         // and idle extra streams cost concurrency to many handles (panels)
-        if (K >= kSplitFixK && !use_seg_fix(h, P) && !h->fwl_now && !h->stream2) {
+        if (!nf && K >= kSplitFixK && !use_seg_fix(h, P) && !h->fwl_now && !h->stream2) {
             HIPCHK(hipStreamCreateWithFlags(&h->stream2, hipStreamNonBlocking));
             HIPCHK(hipEventCreateWithFlags(&h->fork_ev, hipEventDisableTiming));
             HIPCHK(hipEventCreateWithFlags(&h->join_ev, hipEventDisableTiming));
         }
-        if (P->graph) {
-            (void)hipGraphExecDestroy(P->graph);
-            P->graph = nullptr;
+        if (graph) {
+            (void)hipGraphExecDestroy(graph);
+            graph = nullptr;
         }
         hipGraph_t g = nullptr;
         HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
@@ -3050,11 +3055,11 @@ struct Engine {
         }
         hipError_t e = hipStreamEndCapture(h->stream, &g);
         if (e != hipSuccess) return fail(FEHIP_EHIP, std::string("graph capture failed: ") + hipGetErrorString(e));
-        e = hipGraphInstantiate(&P->graph, g, nullptr, nullptr, 0);
+        e = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (e != hipSuccess) return fail(FEHIP_EHIP, std::string("graph instantiate failed: ") + hipGetErrorString(e));
-        P->graph_iters = M;
-        P->graph_fwl = h->fwl_now;
+        P->graph_iters[nf] = M;
+        P->graph_fwl[nf] = h->fwl_now;
         return 0;
     }
 
@@ -3065,20 +3070,38 @@ struct Engine {
     // back (blocking or not).  Launches after the stop exit at entry.
     struct Run {
         int64_t launched = 0, maxiter = 0;
-        int cur = 0;
+        int cur = 0, Kreal = 0;
+        double tol = 0.0;
+        bool nf = false, fwl = false;  // in level space, projected
     };
 
     static int launch_replay(fehip_solver *h, Plan *P, Run &run, int slot) {
-        HIPCHK(hipGraphLaunch(P->graph, h->stream));
+        HIPCHK(hipGraphLaunch(P->graph[run.nf], h->stream));
         HIPCHK(hipMemcpyAsync(h->h_flag + 1 + slot, P->all_done, sizeof(int32_t), hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipEventRecord(h->poll_ev[slot], h->stream));
-        run.launched += P->graph_iters;
+        run.launched += P->graph_iters[run.nf];
         return 0;
     }
 
     static int lsmr_start(fehip_solver *h, Plan *P, int Kreal, double tol, int64_t maxiter, Run &run) {
         if constexpr (sizeof(T) == 8) CHK(nf_plan(h, P));
-        const bool nf = use_nf(h, P);
+        run = Run{};
+        run.maxiter = maxiter;
+        run.Kreal = Kreal;
+        run.tol = tol;
+        run.nf = use_nf(h, P);
+        run.fwl = h->fwl_now;
+        if (run.nf)
+            hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream,
+                               (const T *)P->x, (T *)P->nx0, h->p * K);
+        return lsmr_begin(h, P, run);
+    }
+
+    static int lsmr_begin(fehip_solver *h, Plan *P, Run &run) {
+        const bool nf = run.nf;
+        const int Kreal = run.Kreal;
+        const double tol = run.tol;
+        const int64_t maxiter = run.maxiter;
         hipLaunchKernelGGL((k_lsmr_setup<Tr>), dim3(1), dim3(64), 0, h->stream, (LsmrState<Tr> *)P->state, K, Kreal,
                            tol, tol, 1e8, maxiter, P->all_done);
         if (h->fwl_now) {
@@ -3102,16 +3125,31 @@ struct Engine {
         }
         CHK(lsmr_vectors(h, P, nf));
         HIPCHK(hipGetLastError());
-        CHK(ensure_graph(h, P));
+        CHK(ensure_graph(h, P, nf));
         // Two replays in flight: while the host waits on replay i's copy of
         // the stop flag, replay i+1 is already queued, so the GPU never
         // drains.  A stop at set-up (b = 0, A'b = 0 or maxiter = 0) makes
         // both exit at entry.
-        run = Run{};
-        run.maxiter = maxiter;
+        run.launched = 0;
+        run.cur = 0;
         CHK(launch_replay(h, P, run, 0));
         CHK(launch_replay(h, P, run, 1));
         return 0;
+    }
+
+    // The solve from its start by the passes over the observations, where level
+    // space cannot tell a column's ||r|| (kNfStartOver): b is in r, x0 in nx0.
+    static int start_over(fehip_solver *h, Plan *P, Run &run) {
+        const bool fwl = h->fwl_now;
+        h->fwl_now = run.fwl;
+        run.nf = false;
+        hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream,
+                           (const T *)P->nx0, (T *)P->x, h->p * K);
+        hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(h->N * K, kBlock)), dim3(kBlock), 0, h->stream, (const T *)P->r,
+                           (T *)P->u, h->N * K);
+        const int rc = lsmr_begin(h, P, run);
+        h->fwl_now = fwl;
+        return rc;
     }
 
     // finished = true once the stop flag is seen (the stream is then idle)
@@ -3125,12 +3163,14 @@ struct Engine {
             if (q != hipSuccess) return fail(FEHIP_EHIP, std::string("event query: ") + hipGetErrorString(q));
         }
         if (h->h_flag[1 + run.cur]) {
-            P->final_copy = h->h_flag[1 + run.cur] - 1;
+            const int flag = h->h_flag[1 + run.cur];
             HIPCHK(hipStreamSynchronize(h->stream));
+            if (flag == kNfStartOver) return start_over(h, P, run);
+            P->final_copy = flag - 1;
             finished = true;
             return 0;
         }
-        if (run.launched > run.maxiter + 3 * P->graph_iters)
+        if (run.launched > run.maxiter + 3 * P->graph_iters[run.nf])
             return fail(FEHIP_EHIP, "LSMR did not reach its stopping rule within maxiter");
         CHK(launch_replay(h, P, run, run.cur));
         run.cur ^= 1;

@@ -52,12 +52,17 @@ struct NormalMat {
     bool stale = false;                      // val does not follow the caches yet
 };
 
+// *all_done where rounding has reached a column's beta: the solve starts over on
+// the observations (see kNfLost).  Else 1 + the state's copy.
+constexpr int32_t kNfStartOver = 4;
+
 // per-column coefficients of the step, written by the scalar launch
 struct NfCols {
     double ia[kMaxK], iold[kMaxK];            // v = ia * w, the one before = iold * wold
     double cq[kMaxK], cv[kMaxK], co[kMaxK];   // w' = cq q + cv w + co wold
     double chb[kMaxK], cx[kMaxK], ch[kMaxK];  // the h / hbar / x update
     double beta1[kMaxK];                      // beta of the iteration before
+    double err[kMaxK];                        // error bound of beta^2
     int32_t on[kMaxK], upd[kMaxK];            // the column runs; an update goes with the step
     int32_t due[kMaxK];                       // alpha and the rotations are due
     int32_t test[kMaxK];                      // the stopping rules are due
@@ -65,6 +70,7 @@ struct NfCols {
     // and x takes the second one back
     double chb2[kMaxK], cx2[kMaxK], ch2[kMaxK];
     int32_t upd2[kMaxK], last[kMaxK], undo[kMaxK];
+    int32_t bad[kMaxK];   // the column asks for a start over (kNfStartOver)
 };
 
 struct NfApply {

@@ -474,13 +474,13 @@ __global__ __launch_bounds__(kBlock) void k_nf_fix_neg(const NfItem *items, int3
 
 // one column's entry of NfCols
 struct ColCoef {
-    double ia, iold, cq, cv, co, chb, cx, ch, beta1, chb2, cx2, ch2;
-    int32_t on, upd, due, test, upd2, last, undo;
+    double ia, iold, cq, cv, co, chb, cx, ch, beta1, chb2, cx2, ch2, err;
+    int32_t on, upd, due, test, upd2, last, undo, bad;
 };
 __device__ __forceinline__ ColCoef load_coef(const NfCols *n, int c) {
     return {n->ia[c],   n->iold[c], n->cq[c],  n->cv[c],   n->co[c],   n->chb[c],  n->cx[c],   n->ch[c],  n->beta1[c],
-            n->chb2[c], n->cx2[c],  n->ch2[c], n->on[c],   n->upd[c],  n->due[c],  n->test[c], n->upd2[c], n->last[c],
-            n->undo[c]};
+            n->chb2[c], n->cx2[c],  n->ch2[c], n->err[c],  n->on[c],   n->upd[c],  n->due[c],  n->test[c], n->upd2[c], n->last[c],
+            n->undo[c], n->bad[c]};
 }
 __device__ __forceinline__ void store_coef(NfCols *n, int c, const ColCoef &f) {
     n->ia[c] = f.ia;
@@ -492,6 +492,7 @@ __device__ __forceinline__ void store_coef(NfCols *n, int c, const ColCoef &f) {
     n->cx[c] = f.cx;
     n->ch[c] = f.ch;
     n->beta1[c] = f.beta1;
+    n->err[c] = f.err;
     n->chb2[c] = f.chb2;
     n->cx2[c] = f.cx2;
     n->ch2[c] = f.ch2;
@@ -502,30 +503,58 @@ __device__ __forceinline__ void store_coef(NfCols *n, int c, const ColCoef &f) {
     n->upd2[c] = f.upd2;
     n->last[c] = f.last;
     n->undo[c] = f.undo;
+    n->bad[c] = f.bad;
 }
+
+// beta^2 = v'Mv - alpha^2 with alpha = ||w'|| / beta of the iteration before: v'Mv
+// carries rounding of a few eps (|v| = 1, M has a unit diagonal), and an error of
+// beta^2 goes on times alpha^2 / beta^2.  A column with noise keeps err / beta^2
+// below 1e-11 (condition numbers to 1e4, 1700 iterations).  It grows to 1 where
+// the FEs explain a column in full, once ||r|| is below about 1e-8 of ||b||, and is
+// there at once for a v in the null space of A (an FE collinear with the
+// eliminated one) or an exhausted Krylov space.  ||A'r|| hangs on the product
+// alpha beta, which stays right, but ||r|| on the betas alone.  A solve whose
+// err / beta^2 passes kNfLost before it stops starts over on the observations,
+// where beta = ||A v - alpha u|| comes from the vectors.
+constexpr double kNfErr = 4.0 * 2.220446049250313e-16, kNfLost = 1e-2;
 
 // alpha and the rotations of the last iteration, from ||w||^2
 __device__ __forceinline__ void rotate_step(LsmrState<double> &s, ColCoef &f, double wsq, int c, ColOps *ops) {
+    const double nw = sqrt(wsq);
     f.iold = f.ia;
-    if (!s.vskip) {
-        const double nw = sqrt(wsq);
-        s.alpha = nw / s.beta;
-        f.ia = nw > 0.0 ? 1.0 / nw : 1.0;
-    }
+    s.alpha = nw / s.beta;
+    f.ia = nw > 0.0 ? 1.0 / nw : 1.0;
     s.inv_alpha = 1.0;
     fin_rotate<double>(s, c, ops);
 }
+// A stopping rule holds whatever ||x|| is (src/utils/lsmr.jl:192-215; ||x||
+// only loosens the two rules on ||r||).
+__device__ __forceinline__ bool stops_anyway(const LsmrState<double> &s) {
+    const double test1 = s.normr / s.normb, test2 = s.normAr / (s.normA * s.normr), test3 = 1.0 / s.condA;
+    return s.iter >= s.maxiter || 1.0 + test3 <= 1.0 || 1.0 + test2 <= 1.0 || 1.0 + test1 <= 1.0 ||
+           test3 <= s.ctol || test2 <= s.atol || test1 <= s.btol;
+}
+
 // beta of this iteration from w'Mw, and w'
 __device__ __forceinline__ void beta_step(LsmrState<double> &s, ColCoef &f, double wMw, int c, ColOps *ops) {
     const double alpha = s.alpha, beta = s.beta;
     const double vMv = wMw * f.ia * f.ia;
     const double co = s.iter == 0 ? 0.0 : -(alpha * beta) * f.iold;
-    const double b2 = fma(-alpha, alpha, vMv);  // beta^2 = v'Mv - alpha^2
-    fin_after_db<double>(s, b2 > 0.0 ? b2 : 0.0, MODE_ITER, c, ops);
+    double b2 = fma(-alpha, alpha, vMv);
+    f.err = kNfErr + (f.due ? f.err * (alpha / beta) * (alpha / beta) : 0.0);
+    if (!(f.err < kNfLost * b2)) {
+        if (!f.due || !stops_anyway(s)) {
+            s.done = f.bad = 1;
+            f.upd = f.upd2 = 0;
+            return;
+        }
+        b2 = b2 > kNfErr ? b2 : kNfErr;  // (it stops where ||x|| is known: nothing hangs on beta)
+    }
+    fin_after_db<double>(s, b2, MODE_ITER, c, ops);
     f.beta1 = beta;
-    f.cq = s.vskip ? 0.0 : f.ia;  // beta = 0: v stays (src/utils/lsmr.jl:106)
-    f.cv = s.vskip ? 1.0 : -vMv * f.ia;
-    f.co = s.vskip ? 0.0 : co;
+    f.cq = f.ia;
+    f.cv = -vMv * f.ia;
+    f.co = co;
     f.on = f.due = 1;
 }
 
@@ -552,14 +581,6 @@ __device__ __forceinline__ void scalar_step(LsmrState<double> &s, ColCoef &f, do
         f.upd = f.test = 1;
     }
     beta_step(s, f, wMw, c, ops);
-}
-
-// A stopping rule holds whatever ||x|| is (src/utils/lsmr.jl:192-215; ||x||
-// only loosens the two rules on ||r||).
-__device__ __forceinline__ bool stops_anyway(const LsmrState<double> &s) {
-    const double test1 = s.normr / s.normb, test2 = s.normAr / (s.normA * s.normr), test3 = 1.0 / s.condA;
-    return s.iter >= s.maxiter || 1.0 + test3 <= 1.0 || 1.0 + test2 <= 1.0 || 1.0 + test1 <= 1.0 ||
-           test3 <= s.ctol || test2 <= s.atol || test1 <= s.btol;
 }
 
 // The same with the updates of iterations j and j + 1 (j odd) in one step,
@@ -693,7 +714,7 @@ __device__ __forceinline__ void scalar_block(const NfScalars &p, ScalarMem<K, NT
     }
     __syncthreads();
 }
-// the result of the launch's workgroup 0; *all_done = 1 + the state's copy
+// the result of the launch's workgroup 0, and *all_done
 template <int K, int NT, bool PAIR>
 __device__ __forceinline__ void scalar_keep(const NfScalars &p, const ScalarMem<K, NT, PAIR> &m) {
     const int c = threadIdx.x;
@@ -706,9 +727,13 @@ __device__ __forceinline__ void scalar_keep(const NfScalars &p, const ScalarMem<
         }
     }
     if (c == 0) {
-        int all = 1;
-        for (int q = 0; q < K; q++) all &= m.state[q].done && !m.coef[q].undo ? 1 : 0;
-        if (all) *p.all_done = 1 + p.copy;
+        int all = 1, bad = 0;
+        for (int q = 0; q < K; q++) {
+            all &= m.state[q].done && !m.coef[q].undo ? 1 : 0;
+            bad |= m.coef[q].bad;
+        }
+        if (bad) *p.all_done = kNfStartOver;
+        else if (all) *p.all_done = 1 + p.copy;
     }
 }
 
@@ -904,8 +929,8 @@ __global__ void k_nf_init_cols(const LsmrState<double> *st, int K, NfCols *cols)
     cols->beta1[c] = 0.0;
     cols->on[c] = c < K && !st[c].done ? 1 : 0;
     cols->upd[c] = cols->due[c] = cols->test[c] = 0;
-    cols->chb2[c] = cols->cx2[c] = cols->ch2[c] = 0.0;
-    cols->upd2[c] = cols->last[c] = cols->undo[c] = 0;
+    cols->chb2[c] = cols->cx2[c] = cols->ch2[c] = cols->err[c] = 0.0;
+    cols->upd2[c] = cols->last[c] = cols->undo[c] = cols->bad[c] = 0;
 }
 
 template <int K>
