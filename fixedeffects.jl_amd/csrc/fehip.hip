@@ -2919,8 +2919,7 @@ struct Engine {
         a.off = m.off;
         a.col = m.col;
         a.val = m.val;
-        a.tile_e = m.tile_e;
-        a.tile_r = m.tile_r;
+        a.tiles = m.tiles;
         a.n0 = a.nt = m.ntile;
         a.w = w;
         a.q = P->nq;

@@ -20,6 +20,13 @@ constexpr int kNfCap = kNfTile + kNfSlack;
 constexpr int kNfRow = 8;       // tile units of one row beside its entries (its vector elements)
 constexpr int kNfRows = kNfCap / kNfRow + 2;  // rows one tile owns, at most
 
+// a tile: its number (ascending with its entries), first entry and the row it
+// is in (the first that begins there, or after it), entries | rows that begin
+// in it << 16
+struct NfTileAt {
+    int32_t k, e0, r0, len_nr;
+};
+
 // a row whose entries lie in several tiles: [t0, t1) hold its later parts,
 // tile t0 - 1 its first
 struct NfItem {
@@ -43,9 +50,8 @@ struct NormalMat {
     int32_t *off = nullptr, *col = nullptr;  // p + 1, nnz
     double *val = nullptr;                   // nnz: sum over the cell of cache_a * cache_b
     std::vector<NfPair> pairs;
-    // tiles: entries [e[k], e[k+1]), rows whose entries start in it [r[k], r[k+1])
     int32_t ntile = 0, ts0 = 0, ts1 = 0;     // [ts0, ts1): the tiles of FE s's rows
-    int32_t *tile_e = nullptr, *tile_r = nullptr;
+    NfTileAt *tiles = nullptr;               // in the order of the launches (FE s's stay in [ts0, ts1))
     NfItem *items = nullptr;
     int32_t nitem = 0, is0 = 0, is1 = 0;     // [is0, is1): the items of FE s's rows
     uint32_t *split = nullptr;               // bit per row: its sum comes from its item
@@ -76,8 +82,8 @@ struct NfCols {
 struct NfApply {
     const int32_t *off, *col;
     const double *val;
-    const int32_t *tile_e, *tile_r;
-    int32_t t0, n0, t1, nt;   // tiles t0 .. t0+n0-1, then t1 .. (nt tiles in all)
+    const NfTileAt *tiles;
+    int32_t t0, n0, t1, nt;   // positions t0 .. t0+n0-1, then t1 .. (nt tiles in all)
     const double *w;          // p x K
     double *q;                // p x K: M w
     double *pa;               // partials [block * K + c]: w'q

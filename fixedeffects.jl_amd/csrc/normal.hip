@@ -97,11 +97,14 @@ __device__ __forceinline__ bool next_tile(const NfApply &p, const TileMap &tm, i
         if (ti < p.nt) break;
     }
     if (ti >= p.nt) return false;
-    d.k = __builtin_amdgcn_readfirstlane(ti < p.n0 ? p.t0 + ti : p.t1 + ti - p.n0);
-    d.e0 = ld_const(p.tile_e, d.k);
-    d.r0 = ld_const(p.tile_r, d.k);
-    d.len = ld_const(p.tile_e, d.k + 1) - d.e0;
-    d.nr = ld_const(p.tile_r, d.k + 1) - d.r0;
+    const int32_t at = __builtin_amdgcn_readfirstlane(ti < p.n0 ? p.t0 + ti : p.t1 + ti - p.n0);
+    const int32_t *q = (const int32_t *)p.tiles;
+    d.k = ld_const(q, 4 * at);
+    d.e0 = ld_const(q, 4 * at + 1);
+    d.r0 = ld_const(q, 4 * at + 2);
+    const int32_t ln = ld_const(q, 4 * at + 3);
+    d.len = ln & 0xffff;
+    d.nr = ln >> 16;
     return true;
 }
 
@@ -1199,6 +1202,22 @@ __global__ void k_nf_tiles(const int32_t *__restrict__ off, int32_t ra, int32_t 
     in[k] = cut;
 }
 
+// first column of each tile
+__global__ void k_nf_tile_cols(const int32_t *__restrict__ te, int32_t nt, const int32_t *__restrict__ col,
+                               int32_t nnz, int32_t *__restrict__ out) {
+    const int32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < nt) out[k] = te[k] < nnz ? col[te[k]] : 0;
+}
+
+// order == nullptr: the tiles' own
+__global__ void k_nf_tile_list(const int32_t *__restrict__ te, const int32_t *__restrict__ tr, int32_t nt,
+                               const int32_t *__restrict__ order, NfTileAt *__restrict__ out) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nt) return;
+    const int32_t k = order ? order[i] : i;
+    out[i] = {k, te[k], tr[k], (te[k + 1] - te[k]) | (tr[k + 1] - tr[k]) << 16};
+}
+
 __global__ void k_nf_split_bits(const NfItem *__restrict__ items, int32_t n, uint32_t *__restrict__ split) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) atomicOr(&split[items[i].row >> 5], 1u << (items[i].row & 31));
@@ -1242,10 +1261,43 @@ void nf_free(fehip_solver *h, NormalMat &m) {
     for (NfPair &q : m.pairs)
         for (void *x : {(void *)q.order, (void *)q.start, (void *)q.dsta, (void *)q.dstb, (void *)q.big})
             solver_free(h, x);
-    for (void *x : {(void *)m.off, (void *)m.col, (void *)m.val, (void *)m.tile_e, (void *)m.tile_r, (void *)m.items,
+    for (void *x : {(void *)m.off, (void *)m.col, (void *)m.val, (void *)m.tiles, (void *)m.items,
                     (void *)m.split})
         solver_free(h, x);
     m = NormalMat{};
+}
+
+// The order in which launches visit the tiles.  A row of many tiles (a year)
+// reads all of v; a few of them one after another read it that often from
+// memory.  Tiles inside such rows are visited by their first column instead, so
+// that the rows' tiles over the same levels run side by side and share an
+// XCD's L2; the others come first, in their own order.  Group after group
+// (bounds), each within itself.
+// Measured (N = 1e7, 20 years): K = 1 48.2 -> 38.2 us a product, K = 32 452 -> 394;
+// 50 years of N = 2e7, K = 16: 357 -> 302.
+constexpr int32_t kNfReorder = 2048;  // fewer tiles: the vectors stay in the L2s anyway
+static std::vector<int32_t> tile_order(const std::vector<int32_t> &in, const std::vector<int32_t> &col, int64_t p,
+                                       const std::vector<int32_t> &bounds) {
+    const int32_t nt = (int32_t)in.size();
+    std::vector<int32_t> order(nt);
+    int shift = 0;
+    while ((p >> shift) >= 1 << 16) shift++;
+    for (size_t g = 0; g + 1 < bounds.size(); g++) {
+        const int32_t a = bounds[g], b = bounds[g + 1];
+        // inside a row: it began before the tile and goes on after it
+        auto inside = [&](int32_t k) { return in[k] >= 0 && k + 1 < b && in[k + 1] == in[k]; };
+        std::vector<int32_t> at((size_t)(p >> shift) + 2, 0);
+        int32_t n = 0;
+        for (int32_t k = a; k < b; k++) {
+            if (inside(k)) at[(col[k] >> shift) + 1]++;
+            else order[a + n++] = k;
+        }
+        at[0] = a + n;
+        for (size_t i = 1; i < at.size(); i++) at[i] += at[i - 1];
+        for (int32_t k = a; k < b; k++)
+            if (inside(k)) order[at[col[k] >> shift]++] = k;
+    }
+    return order;
 }
 
 static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat &m, int *fits) {
@@ -1395,24 +1447,41 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat 
     m.ts0 = (int32_t)nt[0];
     m.ts1 = (int32_t)(nt[0] + nt[1]);
     int32_t *tin = nullptr;
-    NRC(alloc(h, &m.tile_e, m.ntile + 1));
-    NRC(alloc(h, &m.tile_r, m.ntile + 1));
+    int32_t *te = nullptr, *tr = nullptr, *tcol = nullptr;
+    const bool reorder = m.ntile >= kNfReorder;
+    NRC(tmp.get(&te, m.ntile + 1));
+    NRC(tmp.get(&tr, m.ntile + 1));
     NRC(tmp.get(&tin, m.ntile + 1));
+    NRC(alloc(h, &m.tiles, m.ntile));
     int64_t at = 0;
     for (int g3 = 0; g3 < 3; g3++) {
         if (nt[g3])
             hipLaunchKernelGGL(k_nf_tiles, dim3(blocks_for(nt[g3], kBlock)), dim3(kBlock), 0, st,
                                (const int32_t *)m.off, (int32_t)ends[g3], (int32_t)ends[g3 + 1], T, (int32_t)nt[g3],
-                               m.tile_e + at, m.tile_r + at, tin + at);
+                               te + at, tr + at, tin + at);
         at += nt[g3];
     }
     NCHK(hipGetLastError());
     const int32_t last[2] = {(int32_t)m.nnz, (int32_t)p};
-    NCHK(hipMemcpyAsync(m.tile_e + m.ntile, &last[0], sizeof(int32_t), hipMemcpyHostToDevice, st));
-    NCHK(hipMemcpyAsync(m.tile_r + m.ntile, &last[1], sizeof(int32_t), hipMemcpyHostToDevice, st));
-    std::vector<int32_t> hin(m.ntile);
+    NCHK(hipMemcpyAsync(te + m.ntile, &last[0], sizeof(int32_t), hipMemcpyHostToDevice, st));
+    NCHK(hipMemcpyAsync(tr + m.ntile, &last[1], sizeof(int32_t), hipMemcpyHostToDevice, st));
+    std::vector<int32_t> hin(m.ntile), hcol(reorder ? m.ntile : 0);
+    if (reorder) {
+        NRC(tmp.get(&tcol, m.ntile));
+        hipLaunchKernelGGL(k_nf_tile_cols, dim3(blocks_for(m.ntile, kBlock)), dim3(kBlock), 0, st,
+                           (const int32_t *)te, m.ntile, (const int32_t *)m.col, (int32_t)m.nnz, tcol);
+        NCHK(hipMemcpyAsync(hcol.data(), tcol, sizeof(int32_t) * m.ntile, hipMemcpyDeviceToHost, st));
+    }
     NCHK(hipMemcpyAsync(hin.data(), tin, sizeof(int32_t) * m.ntile, hipMemcpyDeviceToHost, st));
     NCHK(hipStreamSynchronize(st));
+    std::vector<int32_t> order;
+    if (reorder) {
+        order = tile_order(hin, hcol, p, {0, m.ts0, m.ts1, m.ntile});
+        NCHK(hipMemcpyAsync(tcol, order.data(), sizeof(int32_t) * m.ntile, hipMemcpyHostToDevice, st));
+    }
+    hipLaunchKernelGGL(k_nf_tile_list, dim3(blocks_for(m.ntile, kBlock)), dim3(kBlock), 0, st, (const int32_t *)te,
+                       (const int32_t *)tr, m.ntile, (const int32_t *)tcol, m.tiles);
+    NCHK(hipGetLastError());
     std::vector<NfItem> items;
     for (int32_t k = 0; k < m.ntile; k++) {
         if (k == m.ts0) m.is0 = (int32_t)items.size();
