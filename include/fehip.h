@@ -54,7 +54,11 @@ typedef struct fehip_mlp fehip_mlp_t;  /* the warm-start network */
                           double_precision = false (src/utils/lsmr.jl:59) */
 #define FEHIP_MIXED 2  /* Float32 streams with segment sums beyond Float32
                           (FP64 sums of exact products, compensated pairs),
-                          Float64 LSMR scalars, Float64 refinement sweeps */
+                          Float64 LSMR scalars, Float64 refinement sweeps.
+                          Solves run in Float64 level space where the handle's
+                          normal matrix is built (at most 6 N entries): an
+                          iteration there takes less time than one over the
+                          Float32 streams */
 
 /* Builds the solver: uploads refs, builds the per-FE CSR permutations on the
  * device, computes scales and caches.
