@@ -53,6 +53,12 @@ PMC_TRAFFIC = {
                                             "profiles/worker_firm_1e7_fp64_k1_csr.md"),
     ("worker_firm_1e7", "fp64", 1, "pieces"): ({"k_fused": 332.4e6, "k_dtx_csr": 103.3e6, "k_update": 88.1e6},
                                                "profiles/worker_firm_1e7_fp64_k1.md"),
+    ("worker_firm_1e7", "fp64", 1, "level"): ({"k_nf_apply": 200.6e6, "k_nf_step": 62.5e6},
+                                              "profiles/worker_firm_1e7_fp64_k1_level.md"),
+    ("worker_firm_1e7_k32", "fp64", 32, "level"): ({"k_nf_apply": 1794.6e6, "k_nf_step": 1975.2e6},
+                                                   "profiles/worker_firm_1e7_fp64_k32_level.md"),
+    ("worker_firm_1e7_k32", "mixed", 32, "level"): ({"k_nf_apply": 1794.6e6, "k_nf_step": 1975.2e6},
+                                                    "profiles/worker_firm_1e7_fp64_k32_level.md"),
     ("worker_firm_1e7_k32", "fp64", 32, "pieces"): ({"k_fused": 6065.9e6, "k_dtx_csr": 1379.6e6,
                                                      "k_update": 2554.9e6}, "profiles/worker_firm_1e7_fp64_k32.md"),
 }

@@ -8,7 +8,7 @@
 // the same bidiagonalization, with the same alpha and beta, and no vector over
 // the observations.  M has a unit diagonal (scale!, src/SolverCPU.jl:78-89) and
 // one entry per pair of levels that meet: a worker/firm/year panel of 1e7
-// observations (1e6 workers, 1e5 firms, 20 years) has 1.4e7 entries, 164 MB,
+// observations (1e6 workers, 1e5 firms, 20 years) has 1.19e7 entries, 142 MB,
 // where the pass over the observations reads and writes 470 MB per column.
 //
 // One iteration is three launches, k counting iterations from 1:
@@ -18,7 +18,9 @@
 //                 beta of k
 //   k_nf_step     x, hbar, h of iteration k-1; the next w; ||x||, ||w||
 // A column that stops does so one product and one scalar launch later than it
-// might; x is the stopping iteration's.
+// might; x is the stopping iteration's.  That is the form with two launches
+// (kNfFolded); with three, x, hbar and h of k-2 and k-1 are updated together in
+// the steps of odd k, and the rules of both are looked at in k+1.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
