@@ -216,6 +216,14 @@ struct FwlScope {
     ~FwlScope() { h->fwl_now = false; }
 };
 
+// A copy on the handle's stream, waited for.  (Not hipMemcpy: on the legacy
+// stream it fails, and ends the capture, while another thread's handle captures.
+// Not hipMemcpyAsync either: from and to pageable memory of a few MB it took
+// milliseconds longer.)
+static hipError_t copy_wait(fehip_solver *h, void *dst, const void *src, size_t bytes, hipMemcpyKind kind) {
+    return hipMemcpyWithStream(dst, src, bytes, kind, h->stream);
+}
+
 template <typename P>
 static int dalloc(fehip_solver *h, P **ptr, size_t count) {
     const size_t bytes = std::max<size_t>(count, 1) * sizeof(P);
@@ -1047,7 +1055,7 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
     for (int g = 0; g < G; g++) {
         FeInfo &f = h->fe[g];
         std::vector<int32_t> o(f.n + 1);
-        HIPCHK(hipMemcpy(o.data(), f.ooff, sizeof(int32_t) * (f.n + 1), hipMemcpyDeviceToHost));
+        HIPCHK(copy_wait(h, o.data(), f.ooff, sizeof(int32_t) * (f.n + 1), hipMemcpyDeviceToHost));
         for (int64_t k = 0; k < f.n; k++)
             if (o[k + 1] - o[k] > kScaleBig) f.big_levels.push_back((int32_t)k);
     }
@@ -2693,7 +2701,7 @@ struct Engine {
         }
         for (auto &e : ev) (void)hipEventDestroy(e);
         int32_t stopped = 0;
-        HIPCHK(hipMemcpy(&stopped, P->all_done, sizeof(int32_t), hipMemcpyDeviceToHost));
+        HIPCHK(copy_wait(h, &stopped, P->all_done, sizeof(int32_t), hipMemcpyDeviceToHost));
         if (stopped) return fail(FEHIP_EHIP, "kernel timing: the filler LSMR stopped early");
         for (int q = 0; q < 8; q++) out_ms[q] = acc[q] / std::max(reps, 1);
         if (!P->csr_blocks && !use_pieces(h, P)) out_ms[2] = 0.0;
@@ -3021,7 +3029,7 @@ struct Engine {
         }
         for (auto &e : ev) (void)hipEventDestroy(e);
         int32_t stopped = 0;
-        HIPCHK(hipMemcpy(&stopped, P->all_done, sizeof(int32_t), hipMemcpyDeviceToHost));
+        HIPCHK(copy_wait(h, &stopped, P->all_done, sizeof(int32_t), hipMemcpyDeviceToHost));
         if (stopped) return fail(FEHIP_EHIP, "kernel timing: the filler LSMR stopped early");
         for (int q = 0; q < 8; q++) out_ms[q] = 0.0;
         const int slot[4] = {0, 1, 6, 7};
@@ -4219,7 +4227,7 @@ int fehip_solve_coefficients(fehip_t *h, const double *y, double tol, int64_t ma
     if (rc == 0) rc = solve_coefficients_dev(h, dy, tol, maxiter, dc, iters, converged);
     if (rc == 0) rc = s_block_to_caller(h, dc);
     for (int g = 0; g < h->G && rc == 0; g++) {
-        hipError_t e = hipMemcpy(coef[g], dc + h->off[g], sizeof(double) * h->n[g], hipMemcpyDeviceToHost);
+        hipError_t e = copy_wait(h, coef[g], dc + h->off[g], sizeof(double) * h->n[g], hipMemcpyDeviceToHost);
         if (e != hipSuccess) rc = fail(FEHIP_EHIP, hipGetErrorString(e));
     }
     dfree(h, dy);
@@ -4471,8 +4479,8 @@ int fehip_get_csr(fehip_t *h, int32_t g, int32_t *perm, int32_t *offsets) {
     if (g == h->s && h->s_int_of) {
         // the blocks of the internal numbering, in caller level order
         std::vector<int32_t> pi(h->N), oi(f.n + 1);
-        HIPCHK(hipMemcpy(pi.data(), f.operm, sizeof(int32_t) * h->N, hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(oi.data(), f.ooff, sizeof(int32_t) * (f.n + 1), hipMemcpyDeviceToHost));
+        HIPCHK(copy_wait(h, pi.data(), f.operm, sizeof(int32_t) * h->N, hipMemcpyDeviceToHost));
+        HIPCHK(copy_wait(h, oi.data(), f.ooff, sizeof(int32_t) * (f.n + 1), hipMemcpyDeviceToHost));
         int32_t at = 0;
         for (int64_t k = 0; k < f.n; k++) {
             const int32_t j = h->h_s_int_of[k];
@@ -4483,8 +4491,8 @@ int fehip_get_csr(fehip_t *h, int32_t g, int32_t *perm, int32_t *offsets) {
         if (offsets) offsets[f.n] = at;
         return 0;
     }
-    if (perm) HIPCHK(hipMemcpy(perm, f.operm, sizeof(int32_t) * h->N, hipMemcpyDeviceToHost));
-    if (offsets) HIPCHK(hipMemcpy(offsets, f.ooff, sizeof(int32_t) * (f.n + 1), hipMemcpyDeviceToHost));
+    if (perm) HIPCHK(copy_wait(h, perm, f.operm, sizeof(int32_t) * h->N, hipMemcpyDeviceToHost));
+    if (offsets) HIPCHK(copy_wait(h, offsets, f.ooff, sizeof(int32_t) * (f.n + 1), hipMemcpyDeviceToHost));
     return 0;
 }
 
@@ -4492,7 +4500,7 @@ int fehip_get_scale(fehip_t *h, int32_t g, double *scale) {
     g_err.clear();
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
     if (g < 0 || g >= h->G || !scale) return fail(FEHIP_EARG, "bad arguments");
-    HIPCHK(hipMemcpy(scale, h->fe[g].scale_d, sizeof(double) * h->fe[g].n, hipMemcpyDeviceToHost));
+    HIPCHK(copy_wait(h, scale, h->fe[g].scale_d, sizeof(double) * h->fe[g].n, hipMemcpyDeviceToHost));
     if (g == h->s && h->s_int_of) {
         const std::vector<double> si(scale, scale + h->fe[g].n);
         for (int64_t k = 0; k < h->fe[g].n; k++) scale[k] = si[h->h_s_int_of[k]];
@@ -4532,8 +4540,8 @@ static int mul_common(fehip_t *h, double *io, const double *other, double a, dou
     CHK(dalloc(h, &dx, h->p));
     const double *y_host = adjoint ? other : io;
     double *x_host = adjoint ? io : (double *)other;
-    HIPCHK(hipMemcpy(dy, y_host, sizeof(double) * h->N, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(dx, x_host, sizeof(double) * h->p, hipMemcpyHostToDevice));
+    HIPCHK(copy_wait(h, dy, y_host, sizeof(double) * h->N, hipMemcpyHostToDevice));
+    HIPCHK(copy_wait(h, dx, x_host, sizeof(double) * h->p, hipMemcpyHostToDevice));
     CHK(s_block_to_internal(h, dx));
     int rc = dispatch(h->precision == FEHIP_MIXED ? FEHIP_FP64 : h->precision, 1, [&](auto e) {
         using E = decltype(e);
@@ -4541,8 +4549,8 @@ static int mul_common(fehip_t *h, double *io, const double *other, double a, dou
     });
     if (rc == 0 && adjoint) rc = s_block_to_caller(h, dx);
     if (rc == 0) {
-        if (adjoint) HIPCHK(hipMemcpy(io, dx, sizeof(double) * h->p, hipMemcpyDeviceToHost));
-        else HIPCHK(hipMemcpy(io, dy, sizeof(double) * h->N, hipMemcpyDeviceToHost));
+        if (adjoint) HIPCHK(copy_wait(h, io, dx, sizeof(double) * h->p, hipMemcpyDeviceToHost));
+        else HIPCHK(copy_wait(h, io, dy, sizeof(double) * h->N, hipMemcpyDeviceToHost));
     }
     dfree(h, dy);
     dfree(h, dx);
