@@ -3072,6 +3072,7 @@ struct Engine {
 
     // LSMR on the columns held in P->u (b) with x as the initial iterate
     // (src/utils/lsmr.jl:46-222); per-column results in the state array.
+    // P->r holds b too, as loaded (raw) or as in u: a start over reads it.
     // lsmr_start queues the set-up and the first two replays of the captured
     // iterations; lsmr_poll advances one replay when its stop flag has come
     // back (blocking or not).  Launches after the stop exit at entry.
@@ -3080,6 +3081,7 @@ struct Engine {
         int cur = 0, Kreal = 0;
         double tol = 0.0;
         bool nf = false, fwl = false;  // in level space, projected
+        bool raw = false;              // r holds b as loaded, not projected
     };
 
     static int launch_replay(fehip_solver *h, Plan *P, Run &run, int slot) {
@@ -3090,12 +3092,14 @@ struct Engine {
         return 0;
     }
 
-    static int lsmr_start(fehip_solver *h, Plan *P, int Kreal, double tol, int64_t maxiter, Run &run) {
+    static int lsmr_start(fehip_solver *h, Plan *P, int Kreal, double tol, int64_t maxiter, Run &run,
+                          bool raw = false) {
         if constexpr (sizeof(T) == 8) CHK(nf_plan(h, P));
         run = Run{};
         run.maxiter = maxiter;
         run.Kreal = Kreal;
         run.tol = tol;
+        run.raw = raw;
         run.nf = use_nf(h, P);
         run.fwl = h->fwl_now;
         if (run.nf)
@@ -3145,7 +3149,8 @@ struct Engine {
     }
 
     // The solve from its start by the passes over the observations, where level
-    // space cannot tell a column's ||r|| (kNfStartOver): b is in r, x0 in nx0.
+    // space cannot tell a column's ||r|| (kNfStartOver): x0 is in nx0, b in r
+    // (of a projected coefficient solve: b before its projection).
     static int start_over(fehip_solver *h, Plan *P, Run &run) {
         const bool fwl = h->fwl_now;
         h->fwl_now = run.fwl;
@@ -3154,6 +3159,7 @@ struct Engine {
                            (const T *)P->nx0, (T *)P->x, h->p * K);
         hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(h->N * K, kBlock)), dim3(kBlock), 0, h->stream, (const T *)P->r,
                            (T *)P->u, h->N * K);
+        if (run.fwl && run.raw) proj_s(h, P, (T *)P->u, MODE_NONE);
         const int rc = lsmr_begin(h, P, run);
         h->fwl_now = fwl;
         return rc;
@@ -3184,9 +3190,9 @@ struct Engine {
         return 0;
     }
 
-    static int lsmr(fehip_solver *h, Plan *P, int Kreal, double tol, int64_t maxiter) {
+    static int lsmr(fehip_solver *h, Plan *P, int Kreal, double tol, int64_t maxiter, bool raw = false) {
         Run run;
-        CHK(lsmr_start(h, P, Kreal, tol, maxiter, run));
+        CHK(lsmr_start(h, P, Kreal, tol, maxiter, run, raw));
         for (bool fin = false; !fin;) CHK(lsmr_poll(h, P, run, true, fin));
         return 0;
     }
@@ -3477,7 +3483,7 @@ struct Engine {
         CHK((get_plan_for<T, Acc, K>(h, &P)));
         const int64_t NK = h->N * K;
         hipLaunchKernelGGL(k_load_cols<T>, dim3(grid_for(NK, kBlock)), dim3(kBlock), 0, h->stream, dy, h->N, K, 1,
-                           h->perm_s, h->sqrtw_int, h->N, (T *)P->u, (T *)nullptr);
+                           h->perm_s, h->sqrtw_int, h->N, (T *)P->r, (T *)P->u);
         hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream, (T *)P->x,
                            h->p * K, (T)0);
         if (coef0) {
@@ -3489,12 +3495,10 @@ struct Engine {
         }
         if (h->fwl_now) {
             // projected: b kept in r; LSMR on (I - A_s A_s') b
-            hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(NK, kBlock)), dim3(kBlock), 0, h->stream, (const T *)P->u,
-                               (T *)P->r, NK);
             CHK(fwl_setup(h, P, 1));
             proj_s(h, P, (T *)P->u, MODE_NONE);
         }
-        CHK(lsmr(h, P, 1, tol, maxiter));
+        CHK(lsmr(h, P, 1, tol, maxiter, true));
         std::vector<int64_t> it;
         std::vector<int> cv;
         CHK(read_state(h, P, 1, it, cv));
