@@ -97,6 +97,7 @@ struct FeInfo {
     std::vector<int32_t> h_ioff;   // host copy of segment offsets (tile schedule)
     std::vector<int32_t> big_levels;  // levels with > kScaleBig observations
     int32_t *d_big = nullptr;
+    double *big_sum = nullptr;  // their sums of z^2 w without scale!'s rounding (weights or interaction; FP64)
 };
 
 struct Plan;  // per-K buffers and schedule
@@ -548,18 +549,23 @@ __global__ void k_scale(const int32_t *__restrict__ off, const int32_t *__restri
 // another, which bounds it, and the other waves put the next 1536 terms into
 // LDS meanwhile (N = 1e7, 20 levels of the year and 1e5 firms: 18.9 and 9.1 ms
 // with one wave that loaded and added in turn, 6.1 and 3.4 now).
+// The loading waves also sum the terms compensated (big_sum, nullptr: not
+// asked for): the serial sum is off by eps sqrt(n) for random terms and by
+// eps n for equal ones (1e6 weights of 0.1: 1.3e-11), which the level-space
+// matrix has on its diagonal (csrc/normal.hip).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_scale_big(const int32_t *__restrict__ off,
                                                       const int32_t *__restrict__ perm,
                                                       const int32_t *__restrict__ levels, const double *__restrict__ w,
                                                       const double *__restrict__ z, T *__restrict__ scale_T,
-                                                      double *__restrict__ scale_d) {
+                                                      double *__restrict__ scale_d, double *__restrict__ big_sum) {
 #pragma clang fp contract(off)
     constexpr int L = kBlock - kWave, B = 8, CH = L * B, A = 16;
     __shared__ double buf[2][CH + 2 * A];
     const int lane = (int)threadIdx.x - kWave;  // of the loading waves
     const int32_t k = levels[blockIdx.x];
     const int32_t q0 = off[k], q1 = off[k + 1];
+    double hi = 0.0, lo = 0.0;  // a loading lane's terms
     auto load = [&](int32_t base, double *out) {
         double t[B];
 #pragma unroll
@@ -575,6 +581,10 @@ __global__ __launch_bounds__(kBlock) void k_scale_big(const int32_t *__restrict_
         }
 #pragma unroll
         for (int j = 0; j < B; j++) out[j * L + lane] = t[j];
+        const double x = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+        const double y = hi + x, xx = y - hi;  // (two-sum)
+        lo += (hi - (y - xx)) + (x - xx);
+        hi = y;
     };
     T s = (T)0;
     int cur = 0;
@@ -611,6 +621,12 @@ __global__ __launch_bounds__(kBlock) void k_scale_big(const int32_t *__restrict_
         scale_T[k] = r;
         scale_d[k] = (double)r;
     }
+    if (!big_sum) return;
+    __shared__ double red[kWavesPerBlock];
+    const double x = column_allreduce<1>(hi + lo);
+    if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = x;
+    __syncthreads();
+    if (threadIdx.x == 0) big_sum[blockIdx.x] = red[1] + (red[2] + red[3]);
 }
 
 // cache[j] = z_i * sqrt(w_i) * scale[ref]  with i = perm_s[j]  (:93)
@@ -688,13 +704,8 @@ static int compute_scale_cache(fehip_solver *h) {
                            h->w_orig, f.z_orig, (T *)f.scale_T[q], f.scale_d);
         HIPCHK(hipGetLastError());
         if (f.big_levels.empty() || (!h->w_orig && !f.z_orig)) continue;
-        if (!f.d_big) {
-            CHK(dalloc(h, &f.d_big, f.big_levels.size()));
-            HIPCHK(hipMemcpyAsync(f.d_big, f.big_levels.data(), sizeof(int32_t) * f.big_levels.size(),
-                                  hipMemcpyHostToDevice, h->stream));
-        }
         hipLaunchKernelGGL(k_scale_big<T>, dim3((unsigned)f.big_levels.size()), dim3(kBlock), 0, h->stream, f.ooff,
-                           f.operm, f.d_big, h->w_orig, f.z_orig, (T *)f.scale_T[q], f.scale_d);
+                           f.operm, f.d_big, h->w_orig, f.z_orig, (T *)f.scale_T[q], f.scale_d, f.big_sum);
         HIPCHK(hipGetLastError());
     }
     for (int g = 0; g < h->G; g++) {
@@ -816,14 +827,22 @@ static NfInput nf_input(const fehip_solver *h) {
     in.off = h->off.data();
     for (int g = 0; g < h->G; g++) {
         in.ref[g] = h->fe[g].ref_int;
-        in.cache[g] = (const double *)h->fe[g].cache_int[0];
+        const FeInfo &f = h->fe[g];
+        in.cache[g] = (const double *)f.cache_int[0];
+        in.big[g] = f.d_big;
+        in.nbig[g] = (int32_t)f.big_levels.size();
+        in.big_sum[g] = h->w_orig || f.z_orig ? f.big_sum : nullptr;
+        in.obs[g] = f.ooff;
+        in.scale[g] = f.scale_d;
     }
     in.stream = h->stream;
     return in;
 }
 
 // the normal matrix follows new caches
-static int refresh_normal(fehip_solver *h) { return h->nf_state == 1 ? nf_values(nf_input(h), h->nf) : 0; }
+static int refresh_normal(fehip_solver *h) {
+    return h->nf_state == 1 ? nf_values(nf_input(h), h->nf, h->nf.projected) : 0;
+}
 
 // Builds the normal matrix of an FP64 handle's fixed effects once
 static int ensure_normal(fehip_solver *h) {
@@ -837,7 +856,7 @@ static int ensure_normal(fehip_solver *h) {
     if (rc == FEHIP_EOOM) return 0;  // the passes over the observations need no more memory
     CHK(rc);
     if (!fits) return 0;
-    CHK(nf_values(in, h->nf));
+    CHK(nf_values(in, h->nf, h->fwl_now));
     HIPCHK(hipStreamSynchronize(h->stream));
     release_spares(h);
     h->nf_state = 1;
@@ -1058,6 +1077,11 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
         HIPCHK(copy_wait(h, o.data(), f.ooff, sizeof(int32_t) * (f.n + 1), hipMemcpyDeviceToHost));
         for (int64_t k = 0; k < f.n; k++)
             if (o[k + 1] - o[k] > kScaleBig) f.big_levels.push_back((int32_t)k);
+        if (f.big_levels.empty()) continue;
+        CHK(dalloc(h, &f.d_big, f.big_levels.size()));
+        HIPCHK(hipMemcpyAsync(f.d_big, f.big_levels.data(), sizeof(int32_t) * f.big_levels.size(),
+                              hipMemcpyHostToDevice, h->stream));
+        if (h->has64 && G > 1) CHK(dalloc(h, &f.big_sum, f.big_levels.size()));
     }
     if (G == 3) {
         int d = -1, g2 = -1;
@@ -2894,6 +2918,11 @@ struct Engine {
 
     static int nf_plan(fehip_solver *h, Plan *P) {
         CHK(ensure_normal(h));
+        if (h->nf_state == 1 && h->nf.projected != h->fwl_now) {
+            // (the values differ in the rows of FE s's large levels)
+            if (h->fe[h->s].big_levels.empty()) h->nf.projected = h->fwl_now;
+            else CHK(nf_values(nf_input(h), h->nf, h->fwl_now));
+        }
         if (h->nf_state != 1 || P->nq) return 0;
         const NormalMat &m = h->nf;
         P->nblocks = nf_apply_blocks(K, m.ntile);

@@ -1,6 +1,6 @@
 // normal.h -- the level-space form of the LSMR iteration: the normal matrix
-// M = A'A of the scaled fixed-effect map (unit diagonal) as one sparse matrix
-// over the levels, and the launches of an iteration that reads M instead of
+// M = A'A of the scaled fixed-effect map (unit diagonal but for rounding) as one
+// sparse matrix over the levels, and the launches of an iteration that reads M instead of
 // the observations.
 #pragma once
 
@@ -55,7 +55,10 @@ struct NormalMat {
     NfItem *items = nullptr;
     int32_t nitem = 0, is0 = 0, is1 = 0;     // [is0, is1): the items of FE s's rows
     uint32_t *split = nullptr;               // bit per row: its sum comes from its item
-    bool stale = false;                      // val does not follow the caches yet
+    // entries on the diagonal, one per large level (NfInput::big), FE after FE
+    int32_t *dpos = nullptr;                 // their places in col and val
+    std::vector<int32_t> dfe;                // G + 1: FE g's are dfe[g] .. dfe[g + 1]
+    bool projected = false;                  // val is the projected iteration's
 };
 
 // *all_done where rounding has reached a column's beta: the solve starts over on
@@ -142,11 +145,18 @@ struct NfInput {
     const int64_t *n = nullptr, *off = nullptr;
     const int32_t *ref[kMaxG] = {};
     const double *cache[kMaxG] = {};
+    // levels of many observations, and the exact sums of z^2 w over them
+    // (nullptr: their counts); every FE's observation offsets and scales
+    const int32_t *big[kMaxG] = {};
+    int32_t nbig[kMaxG] = {};
+    const double *big_sum[kMaxG] = {};
+    const int32_t *obs[kMaxG] = {};
+    const double *scale[kMaxG] = {};
     hipStream_t stream = nullptr;
 };
 // nnz limit for the form to be taken; *fits = 0 leaves m empty
 int nf_build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat &m, int *fits);
-int nf_values(const NfInput &in, NormalMat &m);
+int nf_values(const NfInput &in, NormalMat &m, bool projected);
 void nf_free(fehip_solver *h, NormalMat &m);
 
 }  // namespace fehip

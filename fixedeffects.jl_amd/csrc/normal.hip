@@ -6,8 +6,9 @@
 //   alpha_{k+1} beta_{k+1} v_{k+1} = M v_k - (v_k'M v_k) v_k - alpha_k beta_k v_{k-1},
 //   beta_{k+1}^2 = v_k'M v_k - alpha_k^2,
 // the same bidiagonalization, with the same alpha and beta, and no vector over
-// the observations.  M has a unit diagonal (scale!, src/SolverCPU.jl:78-89) and
-// one entry per pair of levels that meet: a worker/firm/year panel of 1e7
+// the observations.  M has a unit diagonal but for scale!'s rounding
+// (src/SolverCPU.jl:78-89; large levels have an entry for what it leaves, see
+// k_nf_diag) and one entry per pair of levels that meet: a worker/firm/year panel of 1e7
 // observations (1e6 workers, 1e5 firms, 20 years) has 1.19e7 entries, 142 MB,
 // where the pass over the observations reads and writes 470 MB per column.
 //
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(kBlock) void k_nf_apply1(NfApply p) {
                 if (NEG) {
                     if (!part) p.neg[r] = -sum;
                 } else {
-                    const double qv = wv + sum;  // (M has a unit diagonal)
+                    const double qv = wv + sum;  // (the diagonal's 1; k_nf_diag)
                     acc += wv * qv;
                     if (!part) p.q[r] = qv;
                 }
@@ -334,7 +335,7 @@ __global__ __launch_bounds__(kBlock) void k_nf_apply(NfApply p) {
             if (!part) st2(p.neg, at, make_double2(-s.s0, -s.s1));
             return;
         }
-        const double q0 = w.x + s.s0, q1 = w.y + s.s1;  // (M has a unit diagonal)
+        const double q0 = w.x + s.s0, q1 = w.y + s.s1;  // (the diagonal's 1; k_nf_diag)
         aq0 += w.x * q0;
         aq1 += w.y * q1;
         if (!part) st2(p.q, at, make_double2(q0, q1));
@@ -512,16 +513,17 @@ __device__ __forceinline__ void store_coef(NfCols *n, int c, const ColCoef &f) {
 }
 
 // beta^2 = v'Mv - alpha^2 with alpha = ||w'|| / beta of the iteration before: v'Mv
-// carries rounding of a few eps (|v| = 1, M has a unit diagonal), and an error of
-// beta^2 goes on times alpha^2 / beta^2.  A column with noise keeps err / beta^2
-// below 1e-11 (condition numbers to 1e4, 1700 iterations).  It grows to 1 where
-// the FEs explain a column in full, once ||r|| is below about 1e-8 of ||b||, and is
+// carries rounding of a few eps (|v| = 1; the diagonal's 1 is off by up to n eps / 4
+// for n = 128 equal observations, the largest level without an entry of its own),
+// and an error of beta^2 goes on times alpha^2 / beta^2.  A column with noise keeps
+// err / beta^2 below 1e-10 (condition numbers to 1e4, 1700 iterations).  It grows to 1
+// where the FEs explain a column in full, once ||r|| is below about 1e-7 of ||b||, and is
 // there at once for a v in the null space of A (an FE collinear with the
 // eliminated one) or an exhausted Krylov space.  ||A'r|| hangs on the product
 // alpha beta, which stays right, but ||r|| on the betas alone.  A solve whose
 // err / beta^2 passes kNfLost before it stops starts over on the observations,
 // where beta = ||A v - alpha u|| comes from the vectors.
-constexpr double kNfErr = 4.0 * 2.220446049250313e-16, kNfLost = 1e-2;
+constexpr double kNfErr = 16.0 * 2.220446049250313e-16, kNfLost = 1e-2;
 
 // alpha and the rotations of the last iteration, from ||w||^2
 __device__ __forceinline__ void rotate_step(LsmrState<double> &s, ColCoef &f, double wsq, int c, ColOps *ops) {
@@ -1173,6 +1175,59 @@ __global__ __launch_bounds__(kBlock) void k_nf_big_values(const int32_t *__restr
     }
 }
 
+// What scale!'s sum leaves on M's diagonal, per large level: its sum rounds once
+// per observation (1e6 weights of 0.1: d = 1 + 1.3e-11), too much for beta^2 =
+// v'Mv - alpha^2 to carry.  An entry at the row's end holds d - 1; levels of fewer
+// observations are within kNfErr.
+__global__ void k_nf_add_diag(const int32_t *__restrict__ big, int32_t n, uint32_t *__restrict__ rows) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) rows[big[i]] += 1;
+}
+
+// (after every pair's entries: cur is at the row's last)
+__global__ void k_nf_place_diag(const int32_t *__restrict__ big, int32_t n, const uint32_t *__restrict__ cur,
+                                int32_t row0, int32_t *__restrict__ dpos, int32_t *__restrict__ col) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int32_t d = (int32_t)cur[big[i]];
+    dpos[i] = d;
+    col[d] = row0 + big[i];
+}
+
+// scale^2 times the sum, less 1
+__device__ __forceinline__ double diag_rest(const double *sum, int32_t i, const int32_t *obs, const double *scale,
+                                            int32_t k) {
+    const double s = sum ? sum[i] : (double)(obs[k + 1] - obs[k]), r = scale[k];
+    return s > 0.0 && s <= 1.7976931348623157e308 ? fma(r, r * s, -1.0) : 0.0;  // (not a sum that overflowed)
+}
+
+__global__ void k_nf_diag(const int32_t *__restrict__ big, int32_t n, const double *__restrict__ sum,
+                          const int32_t *__restrict__ obs, const double *__restrict__ scale, int32_t row0,
+                          const int32_t *__restrict__ dpos, int32_t *__restrict__ col, double *__restrict__ val) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    col[dpos[i]] = row0 + big[i];
+    val[dpos[i]] = diag_rest(sum, i, obs, scale, big[i]);
+}
+
+// The rows of FE s in the projected iteration, a workgroup per large level: they
+// form (A_s'A_s)^-1 A_s'A_o v, so their entries are divided by d; the one on the
+// diagonal is taken out (its element of v is being written by the same launch).
+__global__ __launch_bounds__(kBlock) void k_nf_project_rows(const int32_t *__restrict__ big,
+                                                            const double *__restrict__ sum,
+                                                            const int32_t *__restrict__ obs,
+                                                            const double *__restrict__ scale,
+                                                            const int32_t *__restrict__ off,
+                                                            int32_t *__restrict__ col, double *__restrict__ val) {
+    const int32_t i = blockIdx.x, k = big[i], e0 = off[k], e1 = off[k + 1] - 1;
+    const double f = 1.0 / (1.0 + diag_rest(sum, i, obs, scale, k));
+    for (int32_t e = e0 + threadIdx.x; e < e1; e += kBlock) val[e] *= f;
+    if (threadIdx.x == 0) {
+        col[e1] = col[e0];
+        val[e1] = 0.0;
+    }
+}
+
 // Tile starts of rows [ra, rb): every T units (an entry is one, a row kNfRow
 // more).  A boundary goes to the end of the row it falls into when at most
 // kNfSlack units of it are left, else it cuts the row (in[k] = that row).
@@ -1264,7 +1319,7 @@ void nf_free(fehip_solver *h, NormalMat &m) {
         for (void *x : {(void *)q.order, (void *)q.start, (void *)q.dsta, (void *)q.dstb, (void *)q.big})
             solver_free(h, x);
     for (void *x : {(void *)m.off, (void *)m.col, (void *)m.val, (void *)m.tiles, (void *)m.items,
-                    (void *)m.split})
+                    (void *)m.split, (void *)m.dpos})
         solver_free(h, x);
     m = NormalMat{};
 }
@@ -1315,6 +1370,12 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat 
     NRC(tmp.get(&count, 1));
     int64_t cells = 0;
     std::vector<int64_t> fe_nnz(in.G, 0);
+    m.dfe.assign(1, 0);
+    for (int g = 0; g < in.G; g++) {
+        fe_nnz[g] = in.nbig[g];
+        m.dfe.push_back(m.dfe.back() + in.nbig[g]);
+    }
+    const int32_t ndiag = m.dfe.back();
     for (int x = 0; x < in.G; x++)
         for (int y = x + 1; y < in.G; y++) {
             // a: FE s where it is one of the two (the internal order keeps its levels together), else the larger
@@ -1356,7 +1417,7 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat 
             cells += nc;
             fe_nnz[a] += nc;
             fe_nnz[b] += nc;
-            if (2 * cells > nnz_max || 2 * cells + (int64_t)kNfRow * p > INT32_MAX) {
+            if (2 * cells > nnz_max || 2 * cells + ndiag + (int64_t)kNfRow * p > INT32_MAX) {
                 *fits = 0;
                 return 0;
             }
@@ -1398,8 +1459,8 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat 
             }
             tmp.drop(list);
         }
-    // rows: the entries of every pair a level takes part in, pair after pair
-    m.nnz = 2 * cells;
+    // rows: the entries of every pair a level takes part in, pair after pair, and a large level's diagonal
+    m.nnz = 2 * cells + ndiag;
     uint32_t *cur = nullptr;
     NRC(tmp.get(&cur, p + 1));
     NRC(alloc(h, &m.off, p + 1));
@@ -1414,6 +1475,10 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat 
         add(ps[i].offa, m.pairs[i].a);
         add(ps[i].offb, m.pairs[i].b);
     }
+    for (int g = 0; g < in.G; g++)
+        if (in.nbig[g])
+            hipLaunchKernelGGL(k_nf_add_diag, dim3(blocks_for(in.nbig[g], kBlock)), dim3(kBlock), 0, st, in.big[g],
+                               in.nbig[g], cur + in.off[g]);
     NCHK(hipGetLastError());
     NRC(solver_scan(h, cur, p, (uint32_t *)m.off));
     NCHK(hipMemcpyAsync(cur, m.off, sizeof(uint32_t) * p, hipMemcpyDeviceToDevice, st));
@@ -1433,6 +1498,12 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat 
         add(w.offb, q.b);
         NCHK(hipGetLastError());
     }
+    NRC(alloc(h, &m.dpos, ndiag));
+    for (int g = 0; g < in.G; g++)
+        if (in.nbig[g])
+            hipLaunchKernelGGL(k_nf_place_diag, dim3(blocks_for(in.nbig[g], kBlock)), dim3(kBlock), 0, st, in.big[g],
+                               in.nbig[g], (const uint32_t *)cur + in.off[g], (int32_t)in.off[g], m.dpos + m.dfe[g], m.col);
+    NCHK(hipGetLastError());
     // tiles: of the FEs before s, of s, of those after it
     // (small problems: shorter tiles, down to a wave's two loads per lane, so that
     // every CU has some)
@@ -1517,7 +1588,7 @@ int nf_build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat &m, 
     return rc;
 }
 
-int nf_values(const NfInput &in, NormalMat &m) {
+int nf_values(const NfInput &in, NormalMat &m, bool projected) {
     for (const NfPair &q : m.pairs) {
         const double *ca = in.cache[q.a], *cb = in.cache[q.b];
         hipLaunchKernelGGL(k_nf_cell_values, dim3(blocks_for(q.ncell, kBlock)), dim3(kBlock), 0, in.stream,
@@ -1528,6 +1599,19 @@ int nf_values(const NfInput &in, NormalMat &m) {
                                (const int32_t *)q.big, (const int32_t *)q.start, (const int32_t *)q.order, ca, cb,
                                (const int32_t *)q.dsta, (const int32_t *)q.dstb, m.val);
     }
+    for (int g = 0; g < in.G; g++) {
+        const int32_t n = in.nbig[g];
+        if (!n) continue;
+        if (projected && g == in.s)
+            hipLaunchKernelGGL(k_nf_project_rows, dim3((unsigned)n), dim3(kBlock), 0, in.stream, in.big[g],
+                               in.big_sum[g], in.obs[g], in.scale[g], (const int32_t *)m.off + in.off[g], m.col,
+                               m.val);
+        else
+            hipLaunchKernelGGL(k_nf_diag, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, in.stream, in.big[g], n,
+                               in.big_sum[g], in.obs[g], in.scale[g], (int32_t)in.off[g],
+                               (const int32_t *)m.dpos + m.dfe[g], m.col, m.val);
+    }
+    m.projected = projected;
     NCHK(hipGetLastError());
     return 0;
 }
