@@ -2095,6 +2095,42 @@ __global__ __launch_bounds__(kFinBlock) void k_col_rms(const T *__restrict__ b, 
 // ---------------------------------------------------------------------------
 // engine: launches of one precision / column count
 // ---------------------------------------------------------------------------
+// some columns of a batch
+struct ColList {
+    int32_t n = 0;
+    int32_t c[kMaxK] = {};
+};
+
+// b (K2 columns) = columns l of a (K), the rest 0
+template <typename T>
+__global__ void k_pick_cols(const T *__restrict__ a, int K, int64_t rows, ColList l, int K2, T *__restrict__ b) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= rows * K2) return;
+    const int64_t r = e / K2;
+    const int i = (int)(e - r * K2);
+    b[e] = i < l.n ? a[r * K + l.c[i]] : (T)0;
+}
+
+// columns l of a (K) = b (K2 columns)
+template <typename T>
+__global__ void k_put_cols(const T *__restrict__ b, int K2, int64_t rows, ColList l, int K, T *__restrict__ a) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= rows * l.n) return;
+    const int64_t r = e / l.n;
+    const int i = (int)(e - r * l.n);
+    a[r * K + l.c[i]] = b[r * K2 + i];
+}
+
+template <typename Tr>
+__global__ void k_put_states(const LsmrState<Tr> *__restrict__ b, ColList l, LsmrState<Tr> *__restrict__ a) {
+    const int i = threadIdx.x;
+    if (i < l.n) a[l.c[i]] = b[i];
+}
+
+template <typename T, typename Acc, typename Tr, typename F>
+static int for_K(int K, F &&f);
+static int padded_K(int K);
+
 template <typename T, typename Acc, typename Tr, int K>
 struct Engine {
     using TT = T;
@@ -3111,6 +3147,7 @@ struct Engine {
         double tol = 0.0;
         bool nf = false, fwl = false;  // in level space, projected
         bool raw = false;              // r holds b as loaded, not projected
+        std::function<int(bool, bool &)> rest;  // columns that started over: lsmr_poll of theirs
     };
 
     static int launch_replay(fehip_solver *h, Plan *P, Run &run, int slot) {
@@ -3177,26 +3214,84 @@ struct Engine {
         return 0;
     }
 
-    // The solve from its start by the passes over the observations, where level
-    // space cannot tell a column's ||r|| (kNfStartOver): x0 is in nx0, b in r
-    // (of a projected coefficient solve: b before its projection).
-    static int start_over(fehip_solver *h, Plan *P, Run &run) {
+    // The columns that level space has lost (NfCols::bad) from their start by the
+    // passes over the observations: x0 is in nx0, b in r (of a projected
+    // coefficient solve: b before its projection).  Up to half of the batch, they
+    // go into a batch of their own width and the others keep their results; more
+    // of them, or no room for that batch's buffers, and the whole batch starts over.
+    static int start_over(fehip_solver *h, Plan *P, Run &run, int copy) {
+        NfCols cols;
+        HIPCHK(copy_wait(h, &cols, P->ncols + copy, sizeof(cols), hipMemcpyDeviceToHost));
+        ColList bad;
+        for (int c = 0; c < run.Kreal; c++)
+            if (cols.bad[c]) bad.c[bad.n++] = c;
         const bool fwl = h->fwl_now;
         h->fwl_now = run.fwl;
-        run.nf = false;
-        hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream,
-                           (const T *)P->nx0, (T *)P->x, h->p * K);
-        hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(h->N * K, kBlock)), dim3(kBlock), 0, h->stream, (const T *)P->r,
-                           (T *)P->u, h->N * K);
-        if (run.fwl && run.raw) proj_s(h, P, (T *)P->u, MODE_NONE);
-        const int rc = lsmr_begin(h, P, run);
+        int rc = FEHIP_EOOM;
+        if (2 * bad.n <= run.Kreal)
+            rc = for_K<T, Acc, Tr>(padded_K(bad.n), [&](auto e) {
+                using E2 = decltype(e);
+                Plan *P2 = nullptr;
+                CHK((get_plan_for<T, Acc, E2::width>(h, &P2)));
+                auto r2 = std::make_shared<typename E2::Run>();
+                CHK(E2::template begin_columns<K>(h, P2, P, bad, run, *r2));
+                P->final_copy = copy;
+                run.rest = [h, P, P2, bad, r2](bool block, bool &finished) {
+                    CHK(E2::lsmr_poll(h, P2, *r2, block, finished));
+                    if (finished) CHK(E2::template end_columns<K>(h, P2, P, bad));
+                    return 0;
+                };
+                return 0;
+            });
+        if (rc == FEHIP_EOOM) {
+            g_err.clear();
+            run.nf = false;
+            hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream,
+                               (const T *)P->nx0, (T *)P->x, h->p * K);
+            hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(h->N * K, kBlock)), dim3(kBlock), 0, h->stream,
+                               (const T *)P->r, (T *)P->u, h->N * K);
+            if (run.fwl && run.raw) proj_s(h, P, (T *)P->u, MODE_NONE);
+            rc = lsmr_begin(h, P, run);
+        }
         h->fwl_now = fwl;
         return rc;
     }
 
-    // finished = true once the stop flag is seen (the stream is then idle)
+    static constexpr int width = K;
+
+    // columns l of a solve of K1 (plan P1) begin on the observations as a batch of this width
+    template <int K1, typename R1>
+    static int begin_columns(fehip_solver *h, Plan *P, const Plan *P1, const ColList &l, const R1 &first, Run &run) {
+        run.maxiter = first.maxiter;
+        run.Kreal = l.n;
+        run.tol = first.tol;
+        run.fwl = first.fwl;
+        hipLaunchKernelGGL(k_pick_cols<T>, dim3(grid_for(h->N * K, kBlock)), dim3(kBlock), 0, h->stream,
+                           (const T *)P1->r, K1, h->N, l, K, (T *)P->u);
+        hipLaunchKernelGGL(k_pick_cols<T>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream,
+                           (const T *)P1->nx0, K1, h->p, l, K, (T *)P->x);
+        if (run.fwl) {
+            CHK(fwl_setup(h, P, l.n));
+            if (first.raw) proj_s(h, P, (T *)P->u, MODE_NONE);
+        }
+        return lsmr_begin(h, P, run);
+    }
+
+    // their x and states to their places
+    template <int K1>
+    static int end_columns(fehip_solver *h, const Plan *P, Plan *P1, const ColList &l) {
+        hipLaunchKernelGGL(k_put_cols<T>, dim3(grid_for(h->p * l.n, kBlock)), dim3(kBlock), 0, h->stream,
+                           (const T *)P->x, K, h->p, l, K1, (T *)P1->x);
+        hipLaunchKernelGGL(k_put_states<Tr>, dim3(1), dim3(kWave), 0, h->stream, (const LsmrState<Tr> *)P->state, l,
+                           (LsmrState<Tr> *)(P1->final_copy ? P1->nstate : P1->state));
+        HIPCHK(hipGetLastError());
+        return 0;
+    }
+
+    // finished = true once the stop flag is seen (the stream then has no iteration left)
     static int lsmr_poll(fehip_solver *h, Plan *P, Run &run, bool block, bool &finished) {
         finished = false;
+        if (run.rest) return run.rest(block, finished);
         if (block) {
             HIPCHK(hipEventSynchronize(h->poll_ev[run.cur]));
         } else {
@@ -3207,7 +3302,8 @@ struct Engine {
         if (h->h_flag[1 + run.cur]) {
             const int flag = h->h_flag[1 + run.cur];
             HIPCHK(hipStreamSynchronize(h->stream));
-            if (flag == kNfStartOver) return start_over(h, P, run);
+            if constexpr (sizeof(T) == 8)
+                if (flag >= kNfStartOver) return start_over(h, P, run, flag - kNfStartOver);
             P->final_copy = flag - 1;
             finished = true;
             return 0;

@@ -61,8 +61,9 @@ struct NormalMat {
     bool projected = false;                  // val is the projected iteration's
 };
 
-// *all_done where rounding has reached a column's beta: the solve starts over on
-// the observations (see kNfLost).  Else 1 + the state's copy.
+// *all_done when every column has stopped: 1 + the state's copy, or this + the
+// copy where rounding has reached the betas of some (bad), which start over on
+// the observations (see kNfLost).
 constexpr int32_t kNfStartOver = 4;
 
 // per-column coefficients of the step, written by the scalar launch
@@ -79,7 +80,7 @@ struct NfCols {
     // and x takes the second one back
     double chb2[kMaxK], cx2[kMaxK], ch2[kMaxK];
     int32_t upd2[kMaxK], last[kMaxK], undo[kMaxK];
-    int32_t bad[kMaxK];   // the column asks for a start over (kNfStartOver)
+    int32_t bad[kMaxK];   // the column has to start over (kNfStartOver)
 };
 
 struct NfApply {

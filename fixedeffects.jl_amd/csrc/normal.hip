@@ -520,9 +520,10 @@ __device__ __forceinline__ void store_coef(NfCols *n, int c, const ColCoef &f) {
 // where the FEs explain a column in full, once ||r|| is below about 1e-7 of ||b||, and is
 // there at once for a v in the null space of A (an FE collinear with the
 // eliminated one) or an exhausted Krylov space.  ||A'r|| hangs on the product
-// alpha beta, which stays right, but ||r|| on the betas alone.  A solve whose
-// err / beta^2 passes kNfLost before it stops starts over on the observations,
-// where beta = ||A v - alpha u|| comes from the vectors.
+// alpha beta, which stays right, but ||r|| on the betas alone.  A column whose
+// err / beta^2 passes kNfLost before it stops is left out from there, and starts
+// over on the observations when the others have stopped; there beta =
+// ||A v - alpha u|| comes from the vectors.
 constexpr double kNfErr = 16.0 * 2.220446049250313e-16, kNfLost = 1e-2;
 
 // alpha and the rotations of the last iteration, from ||w||^2
@@ -739,8 +740,7 @@ __device__ __forceinline__ void scalar_keep(const NfScalars &p, const ScalarMem<
             all &= m.state[q].done && !m.coef[q].undo ? 1 : 0;
             bad |= m.coef[q].bad;
         }
-        if (bad) *p.all_done = kNfStartOver;
-        else if (all) *p.all_done = 1 + p.copy;
+        if (all) *p.all_done = (bad ? kNfStartOver : 1) + p.copy;
     }
 }
 
