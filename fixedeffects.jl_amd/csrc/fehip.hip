@@ -200,6 +200,7 @@ struct fehip_solver {
     // many entries)
     NormalMat nf;
     int nf_state = 0;
+    bool nf_busy = false;  // a solve iterates with it (dalloc gives it up for room otherwise)
 };
 
 // With separate CSR and fix-up launches (FEHIP_SEG_FIX=0), from this batch
@@ -225,6 +226,11 @@ static hipError_t copy_wait(fehip_solver *h, void *dst, const void *src, size_t 
     return hipMemcpyWithStream(dst, src, bytes, kind, h->stream);
 }
 
+static void release_spares(fehip_solver *h);
+static void give_up_normal(fehip_solver *h);
+
+// Where the device has no room: the pool is emptied (pool_get), then the
+// handle's spares go, then its normal matrix, which a solve can do without.
 template <typename P>
 static int dalloc(fehip_solver *h, P **ptr, size_t count) {
     const size_t bytes = std::max<size_t>(count, 1) * sizeof(P);
@@ -237,7 +243,15 @@ static int dalloc(fehip_solver *h, P **ptr, size_t count) {
         b = {it->first, it->second.second};
         h->spares.erase(it);
     } else {
-        const hipError_t e = pool_get(bytes, &q, &b.size, &b.device);
+        hipError_t e = pool_get(bytes, &q, &b.size, &b.device);
+        if (e != hipSuccess && !h->spares.empty() && hipStreamSynchronize(h->stream) == hipSuccess) {
+            release_spares(h);
+            e = pool_get(bytes, &q, &b.size, &b.device);
+        }
+        if (e != hipSuccess && h->nf_state == 1 && !h->nf_busy) {
+            give_up_normal(h);
+            e = pool_get(bytes, &q, &b.size, &b.device);
+        }
         if (e != hipSuccess) {
             (void)hipGetLastError();
             return fail(FEHIP_EOOM, "hipMalloc of " + std::to_string(count * sizeof(P)) + " bytes failed: " +
@@ -267,6 +281,16 @@ static void release_spares(fehip_solver *h) {
     h->spares.clear();
 }
 
+// the same at the end of a call that used scratch
+static void settle(fehip_solver *h) {
+    if (h && !h->spares.empty() && hipStreamSynchronize(h->stream) == hipSuccess) release_spares(h);
+}
+// (declared first: it runs when a call's other locals are gone)
+struct Settle {
+    fehip_solver *h;
+    ~Settle() { settle(h); }
+};
+
 static void release_all(fehip_solver *h) {
     for (auto &b : h->allocs) pool_put(b.first, b.second.size, b.second.device);
     h->allocs.clear();
@@ -289,23 +313,6 @@ static inline unsigned grid_for(int64_t n, int per_block) {
 // ---------------------------------------------------------------------------
 // device sort: stable radix sort of (key, index) -> CSR
 // ---------------------------------------------------------------------------
-static int ensure_sort_scratch(fehip_solver *h, int64_t N) {
-    if (h->sort_cap >= N) return 0;
-    for (int b = 0; b < 2; b++) {
-        dfree(h, h->sk[b]);
-        dfree(h, h->sv[b]);
-        CHK(dalloc(h, &h->sk[b], N));
-        CHK(dalloc(h, &h->sv[b], N));
-    }
-    dfree(h, h->hist);
-    dfree(h, h->sums);
-    const int64_t ntiles = (N + kSortTile - 1) / kSortTile;
-    CHK(dalloc(h, &h->hist, 256 * ntiles + 1));
-    CHK(dalloc(h, &h->sums, (256 * ntiles + kSortTile - 1) / kSortTile + 1));
-    h->sort_cap = N;
-    return 0;
-}
-
 static void free_sort_scratch(fehip_solver *h) {
     for (int b = 0; b < 2; b++) {
         dfree(h, h->sk[b]);
@@ -316,6 +323,20 @@ static void free_sort_scratch(fehip_solver *h) {
     dfree(h, h->sums);
     h->hist = h->sums = nullptr;
     h->sort_cap = 0;
+}
+
+static int ensure_sort_scratch(fehip_solver *h, int64_t N) {
+    if (h->sort_cap >= N) return 0;
+    free_sort_scratch(h);
+    for (int b = 0; b < 2; b++) {
+        CHK(dalloc(h, &h->sk[b], N));
+        CHK(dalloc(h, &h->sv[b], N));
+    }
+    const int64_t ntiles = (N + kSortTile - 1) / kSortTile;
+    CHK(dalloc(h, &h->hist, 256 * ntiles + 1));
+    CHK(dalloc(h, &h->sums, (256 * ntiles + kSortTile - 1) / kSortTile + 1));
+    h->sort_cap = N;
+    return 0;
 }
 
 // sums: (n + kSortTile - 1) / kSortTile + 1 entries
@@ -757,10 +778,22 @@ static int do_update_weights(fehip_solver *h, const double *w) {
     if ((w != nullptr) != (h->w_orig != nullptr)) drop_graphs(h);
     if (w) {
         // into a block of its own: the handle stays as it is if they are refused
+        // (where there is no room for one: checked here, then over the old ones)
         double *dw = nullptr;
         unsigned long long *dbad = nullptr, bad = ~0ull;
-        CHK(dalloc(h, &dw, h->N));
-        int rc = dalloc(h, &dbad, 1);
+        int rc = dalloc(h, &dw, h->N);
+        if (rc == FEHIP_EOOM && h->w_orig) {
+            for (int64_t i = 0; i < h->N; i++)
+                if (!(w[i] > 0.0) || !std::isfinite(w[i])) {
+                    bad = (unsigned long long)i;
+                    break;
+                }
+            if (bad == ~0ull) {
+                g_err.clear();
+                HIPCHK(copy_in(h->w_orig, w, sizeof(double) * h->N, h->stream));
+            }
+        }
+        if (rc == 0) rc = dalloc(h, &dbad, 1);
         auto check = [&]() -> int {
             HIPCHK(copy_in(dw, w, sizeof(double) * h->N, h->stream));
             hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, h->stream, dbad, ~0ull);
@@ -769,19 +802,22 @@ static int do_update_weights(fehip_solver *h, const double *w) {
             HIPCHK(hipGetLastError());
             HIPCHK(hipMemcpyAsync(&bad, dbad, sizeof(bad), hipMemcpyDeviceToHost, h->stream));
             HIPCHK(hipStreamSynchronize(h->stream));
-            if (bad != ~0ull)
-                return fail(FEHIP_EARG, "weights must be positive and finite (observation " + std::to_string(bad + 1) +
-                                            ")");
             return 0;
         };
+        const bool over = rc == FEHIP_EOOM && !dw && h->w_orig;
         if (rc == 0) rc = check();
         dfree(h, dbad);
+        if (bad != ~0ull)
+            rc = fail(FEHIP_EARG, "weights must be positive and finite (observation " + std::to_string(bad + 1) + ")");
+        else if (over) rc = 0;
         if (rc) {
             dfree(h, dw);
             return rc;
         }
-        dfree(h, h->w_orig);
-        h->w_orig = dw;
+        if (!over) {
+            dfree(h, h->w_orig);
+            h->w_orig = dw;
+        }
     } else {
         dfree(h, h->w_orig);
         dfree(h, h->sqrtw_int);
@@ -853,13 +889,15 @@ static int ensure_normal(fehip_solver *h) {
     const NfInput in = nf_input(h);
     const int rc = nf_build(h, in, 6 * h->N, h->nf, &fits);
     free_sort_scratch(h);
-    if (rc == FEHIP_EOOM) return 0;  // the passes over the observations need no more memory
-    CHK(rc);
-    if (!fits) return 0;
-    CHK(nf_values(in, h->nf, h->fwl_now));
+    if (rc == 0 && fits) CHK(nf_values(in, h->nf, h->fwl_now));
     HIPCHK(hipStreamSynchronize(h->stream));
     release_spares(h);
-    h->nf_state = 1;
+    if (rc == FEHIP_EOOM) {  // the passes over the observations need no more memory
+        g_err.clear();
+        return 0;
+    }
+    CHK(rc);
+    if (fits) h->nf_state = 1;
     return 0;
 }
 
@@ -1251,6 +1289,7 @@ struct Plan {
     NfCols *ncols = nullptr;
     void *nstate = nullptr;      // the state's second copy (folded scalar steps), or the pair kept for the rules
     bool nfold = false;
+    bool nf_none = false;        // there was no room for them
     int final_copy = 0;          // where the last solve left its state
     double *npa = nullptr, *npx = nullptr, *npw = nullptr, *nhead = nullptr, *ntail = nullptr;
     unsigned nblocks = 0, nstep = 0, nfix = 0;
@@ -1258,6 +1297,9 @@ struct Plan {
 
 static int build_pieces(fehip_solver *h, Plan *P, size_t ts, const std::vector<FixItem> &dense_items,
                         int64_t tiles);
+
+static void destroy_plan(fehip_solver *h, Plan *P);
+static int build_plan(fehip_solver *h, int K, size_t ts, Plan *P, int64_t waves_f, int64_t waves_c);
 
 // waves_f / waves_c: how many waves of the fused pass / of the CSR D'u launch
 // the device holds at once; each gets one tile
@@ -1268,8 +1310,19 @@ static int get_plan(fehip_solver *h, int K, size_t ts, Plan **out, int64_t waves
         *out = it->second;
         return 0;
     }
-    std::unique_ptr<Plan> pl(new Plan());
-    Plan *P = pl.get();
+    Plan *P = new Plan();
+    const int rc = build_plan(h, K, ts, P, waves_f, waves_c);
+    if (rc != 0) {
+        if (h->stream) (void)hipStreamSynchronize(h->stream);
+        destroy_plan(h, P);
+        return rc;
+    }
+    h->plans[key] = P;
+    *out = P;
+    return 0;
+}
+
+static int build_plan(fehip_solver *h, int K, size_t ts, Plan *P, int64_t waves_f, int64_t waves_c) {
     P->K = K;
     const int64_t N = h->N;
     P->waves_f = waves_f;
@@ -1507,8 +1560,6 @@ static int get_plan(fehip_solver *h, int K, size_t ts, Plan **out, int64_t waves
     }
     HIPCHK(hipStreamSynchronize(h->stream));
     release_spares(h);
-    h->plans[key] = pl.release();
-    *out = P;
     return 0;
 }
 
@@ -1759,6 +1810,41 @@ static void drop_graphs(fehip_solver *h) {
             if (g) (void)hipGraphExecDestroy(g);
             g = nullptr;
         }
+}
+
+// a plan's vectors of the level-space iteration
+template <typename P>
+static void dfree_null(fehip_solver *h, P *&ptr) {
+    dfree(h, ptr);
+    ptr = nullptr;
+}
+static void drop_nf_vectors(fehip_solver *h, Plan *P) {
+    dfree_null(h, P->ncols);
+    dfree_null(h, P->nstate);
+    dfree_null(h, P->npa);
+    dfree_null(h, P->npx);
+    dfree_null(h, P->npw);
+    dfree_null(h, P->nhead);
+    dfree_null(h, P->ntail);
+    dfree_null(h, P->nw);
+    dfree_null(h, P->nx0);
+    dfree_null(h, P->nq);
+}
+
+// The normal matrix and what its iterations hold go back to the pool; later
+// solves iterate on the observations.
+static void give_up_normal(fehip_solver *h) {
+    (void)hipStreamSynchronize(h->stream);
+    for (auto &kv : h->plans) {
+        hipGraphExec_t &g = kv.second->graph[1];
+        if (g) (void)hipGraphExecDestroy(g);
+        g = nullptr;
+        drop_nf_vectors(h, kv.second);
+        kv.second->final_copy = 0;
+    }
+    nf_free(h, h->nf);
+    h->nf_state = -1;
+    release_spares(h);
 }
 
 static void destroy_all_plans(fehip_solver *h) {
@@ -2959,12 +3045,27 @@ struct Engine {
             if (h->fe[h->s].big_levels.empty()) h->nf.projected = h->fwl_now;
             else CHK(nf_values(nf_input(h), h->nf, h->fwl_now));
         }
-        if (h->nf_state != 1 || P->nq) return 0;
+        if (h->nf_state != 1 || P->nq || P->nf_none) return 0;
         const NormalMat &m = h->nf;
         P->nblocks = nf_apply_blocks(K, m.ntile);
         P->nfix = (unsigned)std::min(std::max(m.nitem, 1), 1024);
         P->nstep = P->nfix + std::min(grid_for(h->p * K, 4 * kBlock), 1024u);
         P->nfold = nf_folds(K, P->nblocks, P->nstep);
+        h->nf_busy = true;  // (not given up for its own vectors)
+        const int rc = nf_vectors(h, P);
+        h->nf_busy = false;
+        if (rc != FEHIP_EOOM) return rc;
+        // no room: this width iterates on the observations
+        g_err.clear();
+        drop_nf_vectors(h, P);
+        P->nf_none = true;
+        HIPCHK(hipStreamSynchronize(h->stream));
+        release_spares(h);
+        return 0;
+    }
+
+    static int nf_vectors(fehip_solver *h, Plan *P) {
+        const NormalMat &m = h->nf;
         CHK(dalloc(h, &P->ncols, 2));
         CHK(dalloc_bytes(h, &P->nstate, sizeof(LsmrState<double>) * 2 * K));
         CHK(dalloc(h, &P->npa, (size_t)P->nblocks * K));
@@ -3071,6 +3172,7 @@ struct Engine {
         Plan *P = nullptr;
         CHK((get_plan_for<T, Acc, K>(h, &P)));
         CHK(nf_plan(h, P));
+        if (!use_nf(h, P)) return time_kernels(h, reps, out_ms);  // (no room for it)
         const int64_t NK = h->N * K, pK = h->p * K;
         hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(NK, kBlock)), dim3(kBlock), 0, h->stream, (T *)P->u, NK, (T)1);
         hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(pK, kBlock)), dim3(kBlock), 0, h->stream, (T *)P->x, pK, (T)0);
@@ -3166,7 +3268,7 @@ struct Engine {
         run.Kreal = Kreal;
         run.tol = tol;
         run.raw = raw;
-        run.nf = use_nf(h, P);
+        run.nf = h->nf_busy = use_nf(h, P);
         run.fwl = h->fwl_now;
         if (run.nf)
             hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(h->p * K, kBlock)), dim3(kBlock), 0, h->stream,
@@ -3371,6 +3473,7 @@ struct Engine {
         HIPCHK(hipMemcpyAsync(st.data(), P->final_copy ? P->nstate : P->state, sizeof(LsmrState<Tr>) * K,
                               hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
+        h->nf_busy = false;
         h->last_info.assign((size_t)Kreal * 9, 0.0);
         for (int c = 0; c < Kreal; c++) {
             double *o = h->last_info.data() + (size_t)c * 9;
@@ -4174,6 +4277,7 @@ int fehip_create_i32(fehip_t **out, int64_t N, int32_t G, const int32_t *const *
 int fehip_update_weights(fehip_t *h, const double *weights) {
     g_err.clear();
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
+    const Settle settle_at_end{h};
     return do_update_weights(h, weights);
 }
 
@@ -4181,6 +4285,7 @@ int fehip_solve_residuals_device(fehip_t *h, double *dY, int32_t K, int64_t ldY,
                                  int64_t *iters, uint8_t *converged) {
     g_err.clear();
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
+    const Settle settle_at_end{h};
     if (K < 1) return fail(FEHIP_EARG, "K must be >= 1");
     if (!dY) return fail(FEHIP_EARG, "dY is NULL");
     if (ldY < h->N) return fail(FEHIP_EDIM, "ldY < N");
@@ -4301,6 +4406,7 @@ int fehip_solve_residuals_panels_host(fehip_t *const *hs, int32_t npanels, doubl
     for (int32_t i = 0; i < npanels; i++) {
         if (hs[i]) (void)hipStreamSynchronize(hs[i]->stream);
         if (dY[i]) dfree(hs[i], dY[i]);
+        settle(hs[i]);
     }
     return rc;
 }
@@ -4309,6 +4415,7 @@ int fehip_solve_residuals(fehip_t *h, double *const *cols, int32_t K, double tol
                           uint8_t *converged) {
     g_err.clear();
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
+    const Settle settle_at_end{h};
     if (K < 1 || !cols) return fail(FEHIP_EARG, "need K >= 1 columns");
     if (maxiter < 1) return fail(FEHIP_EARG, "maxiter must be >= 1");
     const int bw = max_batch(h);
@@ -4343,6 +4450,7 @@ int fehip_solve_coefficients(fehip_t *h, const double *y, double tol, int64_t ma
                              int64_t *iters, uint8_t *converged) {
     g_err.clear();
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
+    const Settle settle_at_end{h};
     if (!y || !coef) return fail(FEHIP_EARG, "y and coef are required");
     if (maxiter < 0) return fail(FEHIP_EARG, "maxiter must be >= 0");
     double *dy = nullptr, *dc = nullptr;
@@ -4368,6 +4476,7 @@ int fehip_solve_coefficients_full(fehip_t *h, const double *y, double tol, int64
                                   double *const *obs, int64_t *iters, uint8_t *converged) {
     g_err.clear();
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
+    const Settle settle_at_end{h};
     if (!y) return fail(FEHIP_EARG, "y is required");
     if (maxiter < 0) return fail(FEHIP_EARG, "maxiter must be >= 0");
     double *dy = nullptr, *dc = nullptr;
@@ -4447,6 +4556,7 @@ int fehip_group_device_noalloc(int64_t N, int32_t ncols, const int64_t *const *d
 int fehip_normalize(fehip_t *h, double *const *coef) {
     g_err.clear();
     if (!h || !coef) return fail(FEHIP_EARG, "bad arguments");
+    const Settle settle_at_end{h};
     for (int g = 0; g < h->G; g++)
         if (!coef[g]) return fail(FEHIP_EARG, "coef[g] is required for every fixed effect");
     double *dc = nullptr;
@@ -4476,6 +4586,7 @@ int fehip_normalize(fehip_t *h, double *const *coef) {
 int fehip_features(fehip_t *h, const double *y, float *feats, double *coef_ap, double *sigma) {
     g_err.clear();
     if (!h || !y || !feats) return fail(FEHIP_EARG, "bad arguments");
+    const Settle settle_at_end{h};
     double *dy = nullptr, *dca = nullptr;
     CHK(dalloc(h, &dy, h->N));
     CHK(dalloc(h, &dca, h->p));
@@ -4516,6 +4627,7 @@ int fehip_features(fehip_t *h, const double *y, float *feats, double *coef_ap, d
 static int solve_from_common(fehip_t *h, double *const *cols, int32_t K, double tol, int64_t maxiter,
                              const double *const *coef0, fehip_mlp_t *net, int64_t *iters, uint8_t *converged) {
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
+    const Settle settle_at_end{h};
     if (K < 1 || K > kMaxK || !cols) return fail(FEHIP_EARG, "need 1..32 columns");
     if (maxiter < 1) return fail(FEHIP_EARG, "maxiter must be >= 1");
     double *dY = nullptr;
@@ -4559,6 +4671,7 @@ int fehip_solve_residuals_learned_device(fehip_t *h, double *dY, int32_t K, int6
                                          int64_t maxiter, fehip_mlp_t *net, int64_t *iters, uint8_t *converged) {
     g_err.clear();
     if (!h || !net || !dY) return fail(FEHIP_EARG, "bad arguments");
+    const Settle settle_at_end{h};
     if (K < 1 || K > kMaxK) return fail(FEHIP_EARG, "need 1..32 columns");
     if (ldY < h->N) return fail(FEHIP_EDIM, "ldY < N");
     if (maxiter < 1) return fail(FEHIP_EARG, "maxiter must be >= 1");
@@ -4572,6 +4685,7 @@ int fehip_solve_coefficients_x0(fehip_t *h, const double *y, double tol, int64_t
                                 double *const *coef, int64_t *iters, uint8_t *converged) {
     g_err.clear();
     if (!h || !y || !coef) return fail(FEHIP_EARG, "bad arguments");
+    const Settle settle_at_end{h};
     if (maxiter < 0) return fail(FEHIP_EARG, "maxiter must be >= 0");
     double *dy = nullptr, *dc = nullptr;
     CHK(dalloc(h, &dy, h->N));
@@ -4640,6 +4754,7 @@ int fehip_get_scale(fehip_t *h, int32_t g, double *scale) {
 int fehip_get_cache(fehip_t *h, int32_t g, double *cache) {
     g_err.clear();
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
+    const Settle settle_at_end{h};
     if (g < 0 || g >= h->G || !cache) return fail(FEHIP_EARG, "bad arguments");
     double *tmp = nullptr, *tmp2 = nullptr;
     CHK(dalloc(h, &tmp, h->N));
@@ -4663,6 +4778,7 @@ int fehip_get_cache(fehip_t *h, int32_t g, double *cache) {
 static int mul_common(fehip_t *h, double *io, const double *other, double a, double b, bool adjoint) {
     g_err.clear();
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
+    const Settle settle_at_end{h};
     if (!io || !other) return fail(FEHIP_EARG, "bad arguments");
     double *dy = nullptr, *dx = nullptr;
     CHK(dalloc(h, &dy, h->N));
@@ -4706,6 +4822,7 @@ int fehip_lsmr_info(fehip_t *h, int32_t col, double *out) {
 int fehip_time_kernels(fehip_t *h, int32_t K, int32_t reps, double *out_ms) {
     g_err.clear();
     if (!h || !out_ms) return fail(FEHIP_EARG, "bad arguments");
+    const Settle settle_at_end{h};
     if (K < 1 || K > kMaxK || reps < 1) return fail(FEHIP_EARG, "K must be in 1..32 and reps >= 1");
     if (h->precision != FEHIP_FP32 && h->G > 1) {
         CHK(ensure_normal(h));
@@ -4719,6 +4836,7 @@ int fehip_time_kernels(fehip_t *h, int32_t K, int32_t reps, double *out_ms) {
 int fehip_plan_info(fehip_t *h, int32_t K, int32_t fp32_storage, int64_t *out) {
     g_err.clear();
     if (!h || !out) return fail(FEHIP_EARG, "bad arguments");
+    const Settle settle_at_end{h};
     if (K < 1 || K > kMaxK) return fail(FEHIP_EARG, "K must be in 1..32");
     if (fp32_storage ? !h->has32 : !h->has64) return fail(FEHIP_EARG, "the handle has no such storage precision");
     auto fill = [&](Plan *P, int wc) {
@@ -4768,6 +4886,7 @@ int fehip_set_algorithm(fehip_t *h, int32_t algorithm) {
 int fehip_set_schedule(fehip_t *h, int64_t tiles_s, int64_t tiles_c, int32_t fuse_dense, int32_t poll_iters) {
     g_err.clear();
     if (!h) return fail(FEHIP_EARG, "handle is NULL");
+    const Settle settle_at_end{h};
     if (tiles_s < 0 || tiles_c < 0 || tiles_s > (1 << 20) || tiles_c > (1 << 20))
         return fail(FEHIP_EARG, "tile counts must be in 0..2^20 (0 = default)");
     if (fuse_dense < -1 || fuse_dense > 1) return fail(FEHIP_EARG, "fuse_dense must be -1, 0 or 1");
@@ -4783,6 +4902,7 @@ int fehip_set_schedule(fehip_t *h, int64_t tiles_s, int64_t tiles_c, int32_t fus
 int fehip_autotune(fehip_t *h, int32_t K, int32_t reps, double *out) {
     g_err.clear();
     if (!h || !out) return fail(FEHIP_EARG, "bad arguments");
+    const Settle settle_at_end{h};
     if (K < 1 || K > kMaxK || reps < 1) return fail(FEHIP_EARG, "K must be in 1..32 and reps >= 1");
     return dispatch(h->precision, padded_K(K), [&](auto e) { return decltype(e)::autotune(h, reps, out); });
 }

@@ -13,7 +13,9 @@ namespace fehip {
 // A block of at least `bytes` on the current device, and its real size and
 // device (for pool_put).  Its contents are undefined.  Blocks come from those
 // given back before where one of the same size class is there, else from
-// hipMalloc (after emptying the pool if that fails).
+// hipMalloc (after emptying the pool if that fails).  FEHIP_DEVICE_MB in the
+// environment limits what blocks may come to per device, in MB; beyond it a
+// call fails as it does where the device has no room.
 hipError_t pool_get(size_t bytes, void **ptr, size_t *size, int *device);
 
 // Gives a block back.  No work that uses it may be pending on any stream.
@@ -21,6 +23,9 @@ hipError_t pool_get(size_t bytes, void **ptr, size_t *size, int *device);
 void pool_put(void *ptr, size_t size, int device);
 
 constexpr size_t kPoolBytes = size_t(4) << 30;
+
+// Frees the blocks the pool keeps, of every device.
+void pool_trim();
 
 // Pageable host memory to the device: the source has been read when the call
 // returns, the device has it in stream order.  Large copies go through pinned

@@ -4,6 +4,8 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <map>
@@ -17,8 +19,10 @@ namespace {
 
 // Size classes: powers of two up to 64 KB, then steps of an eighth of the
 // power of two below, so a block is at most 1/8 larger than asked for and
-// handles of nearly the same size share blocks.
+// handles of nearly the same size share blocks; from 1 GiB on, steps of 2 MiB
+// (what the device maps), so a handle that fills the device gives little away.
 size_t size_class(size_t b) {
+    if (b >= size_t(1) << 30) return (b + (size_t(2) << 20) - 1) >> 21 << 21;
     if (b <= 256) return 256;
     size_t p = 256;
     while (p * 2 <= b) p *= 2;
@@ -32,14 +36,56 @@ struct Pool {
     std::mutex mu;
     std::multimap<size_t, void *> blocks;
     size_t held = 0;
+    size_t total = 0;  // blocks in use and held
+
+    // hipMalloc and hipFree, counted (mu is not held)
+    hipError_t take(void **ptr, size_t size, size_t limit) {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            if (size > limit || total > limit - size) return hipErrorOutOfMemory;
+            total += size;
+        }
+        const hipError_t e = hipMalloc(ptr, size);
+        if (e == hipSuccess) return e;
+        (void)hipGetLastError();
+        *ptr = nullptr;
+        std::lock_guard<std::mutex> lk(mu);
+        total -= size;
+        return e;
+    }
+    void drop(void *ptr, size_t size) {
+        (void)hipFree(ptr);
+        std::lock_guard<std::mutex> lk(mu);
+        total -= size;
+    }
+    bool over(size_t limit) {
+        std::lock_guard<std::mutex> lk(mu);
+        return total > limit;
+    }
+    void trim() {
+        std::multimap<size_t, void *> out;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            out.swap(blocks);
+            held = 0;
+        }
+        for (auto &b : out) drop(b.second, b.first);
+    }
 };
 
 // one per device, never destroyed (handles may be closed at process exit)
+struct Pools {
+    std::mutex mu;
+    std::map<int, Pool *> by_device;
+};
+Pools &pools() {
+    static Pools *p = new Pools();
+    return *p;
+}
 Pool &pool_of(int device) {
-    static std::mutex mu;
-    static std::map<int, Pool *> *pools = new std::map<int, Pool *>();
-    std::lock_guard<std::mutex> lk(mu);
-    Pool *&p = (*pools)[device];
+    Pools &ps = pools();
+    std::lock_guard<std::mutex> lk(ps.mu);
+    Pool *&p = ps.by_device[device];
     if (!p) p = new Pool();
     return *p;
 }
@@ -52,6 +98,9 @@ hipError_t pool_get(size_t bytes, void **ptr, size_t *size, int *device) {
     if (e != hipSuccess) return e;
     *size = size_class(bytes);
     Pool &p = pool_of(*device);
+    const char *env = getenv("FEHIP_DEVICE_MB");
+    const size_t limit = env && *env ? (size_t)std::max(0ll, atoll(env)) << 20 : SIZE_MAX;
+    if (limit != SIZE_MAX && p.over(limit)) p.trim();
     {
         std::lock_guard<std::mutex> lk(p.mu);
         auto it = p.blocks.find(*size);
@@ -62,19 +111,10 @@ hipError_t pool_get(size_t bytes, void **ptr, size_t *size, int *device) {
             return hipSuccess;
         }
     }
-    e = hipMalloc(ptr, *size);
+    e = p.take(ptr, *size, limit);
     if (e == hipSuccess) return e;
-    (void)hipGetLastError();
-    std::vector<void *> out;
-    {
-        std::lock_guard<std::mutex> lk(p.mu);
-        for (auto &b : p.blocks) out.push_back(b.second);
-        p.blocks.clear();
-        p.held = 0;
-    }
-    for (void *q : out) (void)hipFree(q);
-    *ptr = nullptr;
-    return hipMalloc(ptr, *size);
+    p.trim();
+    return p.take(ptr, *size, limit);
 }
 
 void pool_put(void *ptr, size_t size, int device) {
@@ -87,7 +127,16 @@ void pool_put(void *ptr, size_t size, int device) {
             return;
         }
     }
-    (void)hipFree(ptr);
+    p.drop(ptr, size);
+}
+
+void pool_trim() {
+    std::vector<Pool *> all;
+    {
+        std::lock_guard<std::mutex> lk(pools().mu);
+        for (auto &p : pools().by_device) all.push_back(p.second);
+    }
+    for (Pool *p : all) p->trim();
 }
 
 // ---------------------------------------------------------------------------
