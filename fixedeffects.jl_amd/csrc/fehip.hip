@@ -4917,6 +4917,12 @@ int fehip_dims(const fehip_t *h, int64_t *N, int32_t *G, int64_t *p) {
 
 const char *fehip_last_error(void) { return g_err.c_str(); }
 
+int fehip_trim(void) {
+    g_err.clear();
+    pool_trim();
+    return 0;
+}
+
 void fehip_destroy(fehip_t *h) {
     if (!h) return;
     if (h->stream) (void)hipStreamSynchronize(h->stream);

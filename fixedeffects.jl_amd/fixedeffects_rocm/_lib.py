@@ -62,6 +62,7 @@ EXPORTS = (
     "fehip_dims",
     "fehip_last_error",
     "fehip_destroy",
+    "fehip_trim",
 )
 
 _i64p = C.POINTER(C.c_int64)
@@ -120,6 +121,7 @@ def _load() -> C.CDLL:
     L.fehip_last_error.argtypes = []
     L.fehip_destroy.argtypes = [_vp]
     L.fehip_destroy.restype = None
+    L.fehip_trim.argtypes = []
     _fp = C.POINTER(C.c_float)
     L.fehip_solve_residuals_x0.argtypes = [_vp, C.POINTER(_dp), C.c_int32, C.c_double, C.c_int64, C.POINTER(_dp),
                                            _i64p, _u8p]

@@ -443,6 +443,11 @@ def _outer(method, double_precision, tol, precision=None):
     return double_precision, tol
 
 
+def trim():
+    """Frees the device memory that closed solvers left in the library's pool (at most 4 GiB per device)."""
+    check(lib.fehip_trim())
+
+
 def solve_residuals_panels(solvers, dptrs, Ks, lds, tol: float = 1e-8, maxiter: int = 10_000):
     """Residualize many panels in one call (fehip_solve_residuals_panels):
     panel i has K[i] device-resident columns at dptrs[i] (column c at

@@ -353,8 +353,15 @@ int fehip_dims(const fehip_t *h, int64_t *N, int32_t *G, int64_t *p);
 /* Message for the last failed call on this thread ("" if none). */
 const char *fehip_last_error(void);
 
-/* Frees the handle and its device memory (NULL is a no-op). */
+/* Closes the handle (NULL is a no-op).  Its device memory goes to a pool that
+ * later handles of the process take theirs from; the pool keeps at most 4 GiB
+ * per device and frees the rest. */
 void fehip_destroy(fehip_t *h);
+
+/* Frees the device memory that closed handles left in the pool (no reference
+ * counterpart: its arrays belong to Julia's garbage collector).  The pool is
+ * also emptied when an allocation finds no room. */
+int fehip_trim(void);
 
 #ifdef __cplusplus
 }

@@ -2,10 +2,12 @@
 the library may hold).  Whatever fits without the level-space matrix
 (FEHIP_NORMAL=0) fits with it: the matrix is given up, or its vectors, or a
 batch of columns that start over, and no call keeps another's scratch."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from fixedeffects_rocm import api
+from fixedeffects_rocm import api, device
 from fixedeffects_rocm._lib import FEHIP_EOOM, FehipError
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +85,20 @@ def test_refused_handles_leave_nothing(gpu, monkeypatch):
         assert _fits(api.FixedEffectSolverROCm, fes, w) is None
     monkeypatch.delenv("FEHIP_DEVICE_MB")
     assert np.array_equal(_columns(api.FixedEffectSolverROCm(fes, w), Y[:1])[0], want[0])
+
+
+def test_trim(gpu):
+    hip = device._hip
+    hip.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    fes, w, Y = _panel()
+    _one_batch(fes, w, Y, "fp64")
+    kept = free()
+    api.trim()
+    assert free() - kept >= 8 * N * 8  # at least one batch's columns
+    _one_batch(fes, w, Y, "fp64")
