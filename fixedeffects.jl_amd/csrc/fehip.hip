@@ -196,8 +196,8 @@ struct fehip_solver {
     int32_t cc_nbig = 0;
     double *cc_part = nullptr;    // their partial sums and counts
     // level-space form of the FP64 iteration (normal.h), built at the first
-    // solve: 0 not looked at, 1 built, -1 not taken (FEHIP_NORMAL=0, or too
-    // many entries)
+    // solve: 0 not looked at, 1 built, -1 not taken (FEHIP_NORMAL=0, too many
+    // entries, no room), -2 not built for a narrow batch (takes_level)
     NormalMat nf;
     int nf_state = 0;
     bool nf_busy = false;  // a solve iterates with it (dalloc gives it up for room otherwise)
@@ -868,6 +868,7 @@ static NfInput nf_input(const fehip_solver *h) {
         in.big[g] = f.d_big;
         in.nbig[g] = (int32_t)f.big_levels.size();
         in.big_sum[g] = h->w_orig || f.z_orig ? f.big_sum : nullptr;
+        if (f.kind == KIND_CSR) in.by_level[g] = f.iperm;
         in.obs[g] = f.ooff;
         in.scale[g] = f.scale_d;
     }
@@ -880,16 +881,33 @@ static int refresh_normal(fehip_solver *h) {
     return h->nf_state == 1 ? nf_values(nf_input(h), h->nf, h->nf.projected) : 0;
 }
 
-// Builds the normal matrix of an FP64 handle's fixed effects once
-static int ensure_normal(fehip_solver *h) {
-    if (h->nf_state) return 0;
+// M is taken up to 6 N entries.  An iteration (random refs, weights; passes / level
+// space) near that limit: of one FE of N/10 levels and three of 80 to 100, K = 1
+// 239 / 92 us at N = 4e6 and 679 / 209 at 1.2e7; of three FEs of N/10, N/20 and
+// N/40, K = 1 33 / 21 us at N = 2e5, 212 / 209 at 4e6 and K = 32 1829 / 1131.  More
+// entries were not measured: there the passes stay.
+constexpr int64_t kNfEntries = 6;
+// What costs then are the entries that gather from a vector larger than half an
+// XCD's L2 (far: FEs of more than 2^18 levels).  N = 1.2e7, K = 1 / 2 / 4 / 8 / 32,
+// level space over passes: 2 N far entries 0.62 / 0.57 / 0.51 / 0.43, 4 N (the
+// third FE of 3050 levels) 0.82 / 0.87 / 0.78 / 0.64, 6 N 1.24 / 1.15 / 1.10 / 0.87.
+// Narrow batches stay with the passes beyond the middle of 4 N and 5 N.
+constexpr int kNfWide = 8;
+static int64_t far_limit(const fehip_solver *h, int K) { return K >= kNfWide ? INT64_MAX : h->N * 9 / 2; }
+
+// M is built, and a batch of K iterates with it
+static bool takes_level(const fehip_solver *h, int K) { return h->nf_state == 1 && h->nf.far <= far_limit(h, K); }
+
+// Builds the normal matrix of an FP64 handle's fixed effects once, for a batch of K
+static int ensure_normal(fehip_solver *h, int K) {
+    if (h->nf_state && !(h->nf_state == -2 && K >= kNfWide)) return 0;
     h->nf_state = -1;
     if (h->G < 2 || !h->has64 || !env_int("FEHIP_NORMAL", 1, 0, 1)) return 0;
     int fits = 0;
     const NfInput in = nf_input(h);
-    const int rc = nf_build(h, in, 6 * h->N, h->nf, &fits);
+    const int rc = nf_build(h, in, kNfEntries * h->N, far_limit(h, K), h->nf, &fits);
     free_sort_scratch(h);
-    if (rc == 0 && fits) CHK(nf_values(in, h->nf, h->fwl_now));
+    if (rc == 0 && fits > 0) CHK(nf_values(in, h->nf, h->fwl_now));
     HIPCHK(hipStreamSynchronize(h->stream));
     release_spares(h);
     if (rc == FEHIP_EOOM) {  // the passes over the observations need no more memory
@@ -897,7 +915,7 @@ static int ensure_normal(fehip_solver *h) {
         return 0;
     }
     CHK(rc);
-    if (fits) h->nf_state = 1;
+    if (fits) h->nf_state = fits > 0 ? 1 : -2;
     return 0;
 }
 
@@ -3036,16 +3054,16 @@ struct Engine {
     }
 
     // the level-space iteration (normal.h) is in use: FP64 on a handle that has M
-    static bool use_nf(const fehip_solver *h, const Plan *P) { return sizeof(T) == 8 && h->nf_state == 1 && P->nq; }
+    static bool use_nf(const fehip_solver *h, const Plan *P) { return sizeof(T) == 8 && takes_level(h, K) && P->nq; }
 
     static int nf_plan(fehip_solver *h, Plan *P) {
-        CHK(ensure_normal(h));
+        CHK(ensure_normal(h, K));
         if (h->nf_state == 1 && h->nf.projected != h->fwl_now) {
             // (the values differ in the rows of FE s's large levels)
             if (h->fe[h->s].big_levels.empty()) h->nf.projected = h->fwl_now;
             else CHK(nf_values(nf_input(h), h->nf, h->fwl_now));
         }
-        if (h->nf_state != 1 || P->nq || P->nf_none) return 0;
+        if (!takes_level(h, K) || P->nq || P->nf_none) return 0;
         const NormalMat &m = h->nf;
         P->nblocks = nf_apply_blocks(K, m.ntile);
         P->nfix = (unsigned)std::min(std::max(m.nitem, 1), 1024);
@@ -3841,8 +3859,8 @@ struct Mixed {
                                int64_t *iters, uint8_t *converged) {
         // an FP64 iteration in level space takes less time than one over the
         // FP32 streams, and the second phase would start its Krylov space anew
-        CHK(ensure_normal(h));
-        if (h->G == 1 || h->nf_state == 1)
+        CHK(ensure_normal(h, K));
+        if (h->G == 1 || takes_level(h, K))
             return E64::solve_residuals(h, dY, Kreal, ldY, kMixedLevelTol * tol, maxiter, iters, converged);
         Plan *P32 = nullptr, *P64 = nullptr;
         CHK((get_plan_for<float, F32x2, K>(h, &P32)));
@@ -3865,8 +3883,8 @@ struct Mixed {
 
     static int solve_coefficients(fehip_solver *h, double *dy, double tol, int64_t maxiter, double *dcoef,
                                   int64_t *iters, uint8_t *converged) {
-        CHK(ensure_normal(h));
-        if (h->nf_state == 1)
+        CHK(ensure_normal(h, K));
+        if (takes_level(h, K))
             return E64::solve_coefficients(h, dy, kMixedLevelTol * tol, maxiter, dcoef, iters, converged);
         Plan *P32 = nullptr, *P64 = nullptr;
         CHK((get_plan_for<float, F32x2, K>(h, &P32)));
@@ -4825,8 +4843,8 @@ int fehip_time_kernels(fehip_t *h, int32_t K, int32_t reps, double *out_ms) {
     const Settle settle_at_end{h};
     if (K < 1 || K > kMaxK || reps < 1) return fail(FEHIP_EARG, "K must be in 1..32 and reps >= 1");
     if (h->precision != FEHIP_FP32 && h->G > 1) {
-        CHK(ensure_normal(h));
-        if (h->nf_state == 1)
+        CHK(ensure_normal(h, padded_K(K)));
+        if (takes_level(h, padded_K(K)))
             return for_K<double, double, double>(padded_K(K),
                                                  [&](auto e) { return decltype(e)::time_level(h, reps, out_ms); });
     }

@@ -44,9 +44,11 @@ struct NfPair {
     int32_t nbig = 0;
 };
 constexpr int kNfBigCell = 32;
+constexpr int64_t kNfFarLevels = 1 << 18;  // 2 MB of one column
 
 struct NormalMat {
     int64_t p = 0, nnz = 0;
+    int64_t far = 0;  // entries whose column is of an FE of more than kNfFarLevels levels
     int32_t *off = nullptr, *col = nullptr;  // p + 1, nnz
     double *val = nullptr;                   // nnz: sum over the cell of cache_a * cache_b
     std::vector<NfPair> pairs;
@@ -146,6 +148,7 @@ struct NfInput {
     const int64_t *n = nullptr, *off = nullptr;
     const int32_t *ref[kMaxG] = {};
     const double *cache[kMaxG] = {};
+    const int32_t *by_level[kMaxG] = {};  // positions sorted (stably) by level, where a handle has them
     // levels of many observations, and the exact sums of z^2 w over them
     // (nullptr: their counts); every FE's observation offsets and scales
     const int32_t *big[kMaxG] = {};
@@ -155,8 +158,9 @@ struct NfInput {
     const double *scale[kMaxG] = {};
     hipStream_t stream = nullptr;
 };
-// nnz limit for the form to be taken; *fits = 0 leaves m empty
-int nf_build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat &m, int *fits);
+// the form is taken up to nnz_max entries (*fits = 1; else 0) of which far_max
+// are far (else -1); m is left empty where it is not
+int nf_build(fehip_solver *h, const NfInput &in, int64_t nnz_max, int64_t far_max, NormalMat &m, int *fits);
 int nf_values(const NfInput &in, NormalMat &m, bool projected);
 void nf_free(fehip_solver *h, NormalMat &m);
 

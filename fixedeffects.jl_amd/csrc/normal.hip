@@ -1357,7 +1357,7 @@ static std::vector<int32_t> tile_order(const std::vector<int32_t> &in, const std
     return order;
 }
 
-static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat &m, int *fits) {
+static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, int64_t far_max, NormalMat &m, int *fits) {
     const int64_t N = in.N;
     const hipStream_t st = in.stream;
     const int64_t p = in.off[in.G];
@@ -1390,19 +1390,23 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat 
             const int32_t *ka = in.ref[a], *kb = in.ref[b];
             int32_t *ska = nullptr, *skb = nullptr;
             if (!(a == in.s && b == in.t_sec)) {
-                int32_t *p1 = nullptr, *k1 = nullptr;
+                int32_t *own = nullptr, *k1 = nullptr;
+                const int32_t *p1 = in.by_level[b];
                 NRC(alloc(h, &q.order, N));
-                NRC(tmp.get(&p1, N));
+                if (!p1) NRC(tmp.get(&own, N));
                 NRC(tmp.get(&k1, N));
                 NRC(tmp.get(&ska, N));
                 NRC(tmp.get(&skb, N));
-                NRC(solver_sort(h, in.ref[b], N, in.n[b], ska, p1, nullptr));
+                if (!p1) {
+                    NRC(solver_sort(h, in.ref[b], N, in.n[b], ska, own, nullptr));
+                    p1 = own;
+                }
                 hipLaunchKernelGGL(k_nf_gather, dim3(blocks_for(N, kBlock)), dim3(kBlock), 0, st, in.ref[a], p1, N, k1);
                 NRC(solver_sort(h, k1, N, in.n[a], ska, q.order, p1));
                 hipLaunchKernelGGL(k_nf_gather, dim3(blocks_for(N, kBlock)), dim3(kBlock), 0, st, in.ref[b], q.order,
                                    N, skb);
                 NCHK(hipGetLastError());
-                tmp.drop(p1);
+                if (own) tmp.drop(own);
                 tmp.drop(k1);
                 ka = ska;
                 kb = skb;
@@ -1417,8 +1421,13 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat 
             cells += nc;
             fe_nnz[a] += nc;
             fe_nnz[b] += nc;
+            m.far += (in.n[a] > kNfFarLevels ? nc : 0) + (in.n[b] > kNfFarLevels ? nc : 0);
             if (2 * cells > nnz_max || 2 * cells + ndiag + (int64_t)kNfRow * p > INT32_MAX) {
                 *fits = 0;
+                return 0;
+            }
+            if (m.far > far_max) {
+                *fits = -1;
                 return 0;
             }
             NRC(tmp.get(&w.ca, nc));
@@ -1581,10 +1590,10 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat 
     return 0;
 }
 
-int nf_build(fehip_solver *h, const NfInput &in, int64_t nnz_max, NormalMat &m, int *fits) {
+int nf_build(fehip_solver *h, const NfInput &in, int64_t nnz_max, int64_t far_max, NormalMat &m, int *fits) {
     *fits = 0;
-    const int rc = build(h, in, nnz_max, m, fits);
-    if (rc || !*fits) nf_free(h, m);
+    const int rc = build(h, in, nnz_max, far_max, m, fits);
+    if (rc || *fits <= 0) nf_free(h, m);
     return rc;
 }
 
