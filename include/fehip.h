@@ -56,9 +56,10 @@ typedef struct fehip_mlp fehip_mlp_t;  /* the warm-start network */
                           (FP64 sums of exact products, compensated pairs),
                           Float64 LSMR scalars, Float64 refinement sweeps.
                           Solves run in Float64 level space where the handle's
-                          normal matrix is built (at most 6 N entries): an
+                          normal matrix is taken (at most 6 N entries): an
                           iteration there takes less time than one over the
-                          Float32 streams */
+                          Float32 streams.  They aim at 0.8 of tol there, as
+                          near the exact residual as the two phases ended */
 
 /* Builds the solver: uploads refs, builds the per-FE CSR permutations on the
  * device, computes scales and caches.
@@ -287,7 +288,8 @@ int fehip_lsmr_info(fehip_t *h, int32_t col, double *out);
 /* Test hook (no reference counterpart): the launch plan of K columns in one
  * storage precision (fp32_storage 0: the FP64 streams of FEHIP_FP64 and of
  * FEHIP_MIXED's FP64 phase; 1: the FP32 streams of FEHIP_FP32 and of
- * FEHIP_MIXED's FP32 phase), built if not yet there.
+ * FEHIP_MIXED's FP32 phase), built if not yet there.  It is the plan of the
+ * passes over the observations, also where solves iterate in level space.
  *   out[0] 1 if the few-level FEs are summed inside the fused pass
  *   out[1] positions per fused-pass tile      out[2] fused-pass tiles
  *   out[3] tiles of the D'u passes (all FEs)  out[4] fix-up items
@@ -335,16 +337,20 @@ int fehip_time_kernels(fehip_t *h, int32_t K, int32_t reps, double *out_ms);
  * levels and of the CSR D'u launch (one wave per tile; 0 = sized by
  * occupancy, or FEHIP_TILES_S / FEHIP_TILES_C), few-level FEs accumulated in
  * the fused pass (1), in their own launch (0) or by default (-1), and LSMR
- * iterations per captured graph (0 = keep).  Drops the handle's plans; the
- * next solve rebuilds them.  Results do not depend on the schedule beyond
- * the order of floating-point sums. */
+ * iterations per captured graph (0 = keep).  Solves in level space take only
+ * poll_iters from it, and the tiles for the passes they begin and end with.
+ * Drops the handle's plans; the next solve rebuilds them.  Results do not
+ * depend on the schedule beyond the order of floating-point sums. */
 int fehip_set_schedule(fehip_t *h, int64_t tiles_s, int64_t tiles_c, int32_t fuse_dense, int32_t poll_iters);
 
 /* Autotuner (no reference counterpart): times the launches of one LSMR
  * iteration on K columns of this handle's data (`reps` launches each) under
  * candidate schedules around the occupancy-sized default and keeps the
  * fastest on the handle.  out[6] = {tiles_s, tiles_c, fuse_dense,
- * poll_iters, best ms per iteration, default ms per iteration}. */
+ * poll_iters, best ms per iteration, default ms per iteration}.  Where solves
+ * of K columns iterate in level space, the schedule kept is that of the passes
+ * over the observations (which solves begin and end with, and fall back to),
+ * and both times are the level-space iteration's, which it does not change. */
 int fehip_autotune(fehip_t *h, int32_t K, int32_t reps, double *out);
 
 /* Dimensions of a handle. */
