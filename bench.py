@@ -128,7 +128,8 @@ def kernel_bytes(N, n, kinds, K, s, factored, weighted, plan):
 def level_bytes(panel, K):
     """Algorithmic HBM bytes per launch of the level-space iteration: M = A'A
     has two entries per distinct pair of levels (a column number and a value),
-    its diagonal is 1.  The step writes the next vector from three and updates
+    its diagonal is 1 (the entries for large levels' rounding, at most N/128, are
+    not counted).  The step writes the next vector from three and updates
     h, hbar and x for two iterations in every other launch (the mean; a small
     problem, whose step does the scalar step too, updates them in each)."""
     G, p = len(panel.n), sum(int(k) for k in panel.n)

@@ -517,7 +517,7 @@ __device__ __forceinline__ void store_coef(NfCols *n, int c, const ColCoef &f) {
 // for n = 128 equal observations, the largest level without an entry of its own),
 // and an error of beta^2 goes on times alpha^2 / beta^2.  A column with noise keeps
 // err / beta^2 below 1e-10 (condition numbers to 1e4, 1700 iterations).  It grows to 1
-// where the FEs explain a column in full, once ||r|| is below about 1e-7 of ||b||, and is
+// where the FEs explain a column in full, once ||r|| is between 1e-6 and 1e-8 of ||b||, and is
 // there at once for a v in the null space of A (an FE collinear with the
 // eliminated one) or an exhausted Krylov space.  ||A'r|| hangs on the product
 // alpha beta, which stays right, but ||r|| on the betas alone.  A column whose
