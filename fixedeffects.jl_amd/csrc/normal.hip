@@ -513,7 +513,7 @@ __device__ __forceinline__ void store_coef(NfCols *n, int c, const ColCoef &f) {
 }
 
 // beta^2 = v'Mv - alpha^2 with alpha = ||w'|| / beta of the iteration before: v'Mv
-// carries rounding of a few eps (|v| = 1; the diagonal's 1 is off by up to n eps / 4
+// carries rounding of a few eps (|v| = 1; the diagonal's 1 is off by up to n eps / 8
 // for n = 128 equal observations, the largest level without an entry of its own),
 // and an error of beta^2 goes on times alpha^2 / beta^2.  A column with noise keeps
 // err / beta^2 below 1e-10 (condition numbers to 1e4, 1700 iterations).  It grows to 1
