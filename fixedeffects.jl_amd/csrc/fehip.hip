@@ -95,9 +95,8 @@ struct FeInfo {
     void *cache_int[2] = {nullptr, nullptr};  // N, internal order
     void *cache_csr[2] = {nullptr, nullptr};  // N, CSR order (== cache_int for KIND_SORTED)
     std::vector<int32_t> h_ioff;   // host copy of segment offsets (tile schedule)
-    std::vector<int32_t> big_levels;  // levels with > kScaleBig observations
-    int32_t *d_big = nullptr;
-    double *big_sum = nullptr;  // their sums of z^2 w without scale!'s rounding (weights or interaction; FP64)
+    int32_t big0 = 0, nbig = 0;  // its levels with > kScaleBig observations: big_rows[big0 .. big0 + nbig)
+    bool big_counts = true;      // their big_sum holds the counts
 };
 
 struct Plan;  // per-K buffers and schedule
@@ -118,6 +117,12 @@ struct fehip_solver {
     std::vector<int32_t> h_s_int_of;
     double *s_tmp = nullptr;      // n_s doubles: a permuted FE s block
     std::vector<int64_t> n, off;
+    // levels with > kScaleBig observations, FE after FE, as rows (off[g] + level),
+    // and their sums of z^2 w without scale!'s rounding (FP64)
+    int32_t nbig = 0;
+    int32_t *big_rows = nullptr;
+    double *big_sum = nullptr;
+    std::vector<double> big_n;  // their counts
     hipStream_t stream = nullptr;
     std::vector<FeInfo> fe;
     int32_t *perm_s = nullptr;  // internal position -> caller's observation
@@ -577,14 +582,15 @@ __global__ void k_scale(const int32_t *__restrict__ off, const int32_t *__restri
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_scale_big(const int32_t *__restrict__ off,
                                                       const int32_t *__restrict__ perm,
-                                                      const int32_t *__restrict__ levels, const double *__restrict__ w,
-                                                      const double *__restrict__ z, T *__restrict__ scale_T,
+                                                      const int32_t *__restrict__ rows, int32_t row0,
+                                                      const double *__restrict__ w, const double *__restrict__ z,
+                                                      T *__restrict__ scale_T,
                                                       double *__restrict__ scale_d, double *__restrict__ big_sum) {
 #pragma clang fp contract(off)
     constexpr int L = kBlock - kWave, B = 8, CH = L * B, A = 16;
     __shared__ double buf[2][CH + 2 * A];
     const int lane = (int)threadIdx.x - kWave;  // of the loading waves
-    const int32_t k = levels[blockIdx.x];
+    const int32_t k = rows[blockIdx.x] - row0;
     const int32_t q0 = off[k], q1 = off[k + 1];
     double hi = 0.0, lo = 0.0;  // a loading lane's terms
     auto load = [&](int32_t base, double *out) {
@@ -724,9 +730,19 @@ static int compute_scale_cache(fehip_solver *h) {
         hipLaunchKernelGGL(k_scale<T>, dim3(grid_for(f.n, 64)), dim3(64), 0, h->stream, f.ooff, f.operm, f.n,
                            h->w_orig, f.z_orig, (T *)f.scale_T[q], f.scale_d);
         HIPCHK(hipGetLastError());
-        if (f.big_levels.empty() || (!h->w_orig && !f.z_orig)) continue;
-        hipLaunchKernelGGL(k_scale_big<T>, dim3((unsigned)f.big_levels.size()), dim3(kBlock), 0, h->stream, f.ooff,
-                           f.operm, f.d_big, h->w_orig, f.z_orig, (T *)f.scale_T[q], f.scale_d, f.big_sum);
+        if (!f.nbig) continue;
+        double *sum = q == 0 ? h->big_sum + f.big0 : nullptr;
+        if (!h->w_orig && !f.z_orig) {
+            if (sum && !f.big_counts)
+                HIPCHK(hipMemcpyAsync(sum, h->big_n.data() + f.big0, sizeof(double) * f.nbig, hipMemcpyHostToDevice,
+                                      h->stream));
+            f.big_counts = true;
+            continue;
+        }
+        f.big_counts = false;
+        hipLaunchKernelGGL(k_scale_big<T>, dim3((unsigned)f.nbig), dim3(kBlock), 0, h->stream, f.ooff, f.operm,
+                           (const int32_t *)h->big_rows + f.big0, (int32_t)h->off[g], h->w_orig, f.z_orig,
+                           (T *)f.scale_T[q], f.scale_d, sum);
         HIPCHK(hipGetLastError());
     }
     for (int g = 0; g < h->G; g++) {
@@ -865,13 +881,13 @@ static NfInput nf_input(const fehip_solver *h) {
         in.ref[g] = h->fe[g].ref_int;
         const FeInfo &f = h->fe[g];
         in.cache[g] = (const double *)f.cache_int[0];
-        in.big[g] = f.d_big;
-        in.nbig[g] = (int32_t)f.big_levels.size();
-        in.big_sum[g] = h->w_orig || f.z_orig ? f.big_sum : nullptr;
+        in.nbig[g] = f.nbig;
         if (f.kind == KIND_CSR) in.by_level[g] = f.iperm;
-        in.obs[g] = f.ooff;
-        in.scale[g] = f.scale_d;
     }
+    in.big0_s = h->fe[h->s].big0;
+    in.big_rows = h->big_rows;
+    in.big_sum = h->big_sum;
+    in.scale = (const double *)h->scale_all[0];
     in.stream = h->stream;
     return in;
 }
@@ -1127,17 +1143,29 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
         }
     }
     HIPCHK(hipStreamSynchronize(h->stream));
+    std::vector<int32_t> big_rows;
     for (int g = 0; g < G; g++) {
         FeInfo &f = h->fe[g];
         std::vector<int32_t> o(f.n + 1);
+        f.big0 = (int32_t)big_rows.size();
         HIPCHK(copy_wait(h, o.data(), f.ooff, sizeof(int32_t) * (f.n + 1), hipMemcpyDeviceToHost));
         for (int64_t k = 0; k < f.n; k++)
-            if (o[k + 1] - o[k] > kScaleBig) f.big_levels.push_back((int32_t)k);
-        if (f.big_levels.empty()) continue;
-        CHK(dalloc(h, &f.d_big, f.big_levels.size()));
-        HIPCHK(hipMemcpyAsync(f.d_big, f.big_levels.data(), sizeof(int32_t) * f.big_levels.size(),
-                              hipMemcpyHostToDevice, h->stream));
-        if (h->has64 && G > 1) CHK(dalloc(h, &f.big_sum, f.big_levels.size()));
+            if (o[k + 1] - o[k] > kScaleBig) {
+                big_rows.push_back((int32_t)(h->off[g] + k));
+                h->big_n.push_back((double)(o[k + 1] - o[k]));
+            }
+        f.nbig = (int32_t)big_rows.size() - f.big0;
+    }
+    h->nbig = (int32_t)big_rows.size();
+    if (h->nbig) {
+        CHK(dalloc(h, &h->big_rows, h->nbig));
+        HIPCHK(hipMemcpyAsync(h->big_rows, big_rows.data(), sizeof(int32_t) * h->nbig, hipMemcpyHostToDevice,
+                              h->stream));
+        if (h->has64) {
+            CHK(dalloc(h, &h->big_sum, h->nbig));
+            HIPCHK(hipMemcpyAsync(h->big_sum, h->big_n.data(), sizeof(double) * h->nbig, hipMemcpyHostToDevice,
+                                  h->stream));
+        }
     }
     if (G == 3) {
         int d = -1, g2 = -1;
@@ -3073,7 +3101,7 @@ struct Engine {
         CHK(ensure_normal(h, K));
         if (h->nf_state == 1 && h->nf.projected != h->fwl_now) {
             // (the values differ in the rows of FE s's large levels)
-            if (h->fe[h->s].big_levels.empty()) h->nf.projected = h->fwl_now;
+            if (!h->fe[h->s].nbig) h->nf.projected = h->fwl_now;
             else CHK(nf_values(nf_input(h), h->nf, h->fwl_now));
         }
         if (!takes_level(h, K) || P->nq || P->nf_none) return 0;

@@ -57,9 +57,9 @@ struct NormalMat {
     NfItem *items = nullptr;
     int32_t nitem = 0, is0 = 0, is1 = 0;     // [is0, is1): the items of FE s's rows
     uint32_t *split = nullptr;               // bit per row: its sum comes from its item
-    // entries on the diagonal, one per large level (NfInput::big), FE after FE
+    // entries on the diagonal, one per large level (NfInput::big_rows)
+    int32_t ndiag = 0;
     int32_t *dpos = nullptr;                 // their places in col and val
-    std::vector<int32_t> dfe;                // G + 1: FE g's are dfe[g] .. dfe[g + 1]
     bool projected = false;                  // val is the projected iteration's
 };
 
@@ -149,13 +149,12 @@ struct NfInput {
     const int32_t *ref[kMaxG] = {};
     const double *cache[kMaxG] = {};
     const int32_t *by_level[kMaxG] = {};  // positions sorted (stably) by level, where a handle has them
-    // levels of many observations, and the exact sums of z^2 w over them
-    // (nullptr: their counts); every FE's observation offsets and scales
-    const int32_t *big[kMaxG] = {};
-    int32_t nbig[kMaxG] = {};
-    const double *big_sum[kMaxG] = {};
-    const int32_t *obs[kMaxG] = {};
-    const double *scale[kMaxG] = {};
+    // levels of many observations, FE after FE, and the exact sums of z^2 w over
+    // them; every level's scale (p)
+    int32_t nbig[kMaxG] = {}, big0_s = 0;  // of each FE; FE s's first
+    const int32_t *big_rows = nullptr;
+    const double *big_sum = nullptr;
+    const double *scale = nullptr;
     hipStream_t stream = nullptr;
 };
 // the form is taken up to nnz_max entries (*fits = 1; else 0) of which far_max

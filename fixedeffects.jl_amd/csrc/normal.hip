@@ -1179,48 +1179,46 @@ __global__ __launch_bounds__(kBlock) void k_nf_big_values(const int32_t *__restr
 // per observation (1e6 weights of 0.1: d = 1 + 1.3e-11), too much for beta^2 =
 // v'Mv - alpha^2 to carry.  An entry at the row's end holds d - 1; levels of fewer
 // observations are within kNfErr.
-__global__ void k_nf_add_diag(const int32_t *__restrict__ big, int32_t n, uint32_t *__restrict__ rows) {
+__global__ void k_nf_add_diag(const int32_t *__restrict__ rows, int32_t n, uint32_t *__restrict__ cnt) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) rows[big[i]] += 1;
+    if (i < n) cnt[rows[i]] += 1;
 }
 
 // (after every pair's entries: cur is at the row's last)
-__global__ void k_nf_place_diag(const int32_t *__restrict__ big, int32_t n, const uint32_t *__restrict__ cur,
-                                int32_t row0, int32_t *__restrict__ dpos, int32_t *__restrict__ col) {
+__global__ void k_nf_place_diag(const int32_t *__restrict__ rows, int32_t n, const uint32_t *__restrict__ cur,
+                                int32_t *__restrict__ dpos, int32_t *__restrict__ col) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int32_t d = (int32_t)cur[big[i]];
+    const int32_t d = (int32_t)cur[rows[i]];
     dpos[i] = d;
-    col[d] = row0 + big[i];
+    col[d] = rows[i];
 }
 
 // scale^2 times the sum, less 1
-__device__ __forceinline__ double diag_rest(const double *sum, int32_t i, const int32_t *obs, const double *scale,
-                                            int32_t k) {
-    const double s = sum ? sum[i] : (double)(obs[k + 1] - obs[k]), r = scale[k];
+__device__ __forceinline__ double diag_rest(double s, double r) {
     return s > 0.0 && s <= 1.7976931348623157e308 ? fma(r, r * s, -1.0) : 0.0;  // (not a sum that overflowed)
 }
 
-__global__ void k_nf_diag(const int32_t *__restrict__ big, int32_t n, const double *__restrict__ sum,
-                          const int32_t *__restrict__ obs, const double *__restrict__ scale, int32_t row0,
+// all but the levels [skip0, skip1) of the list
+__global__ void k_nf_diag(const int32_t *__restrict__ rows, int32_t n, int32_t skip0, int32_t skip1,
+                          const double *__restrict__ sum, const double *__restrict__ scale,
                           const int32_t *__restrict__ dpos, int32_t *__restrict__ col, double *__restrict__ val) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    col[dpos[i]] = row0 + big[i];
-    val[dpos[i]] = diag_rest(sum, i, obs, scale, big[i]);
+    if (i >= n || (i >= skip0 && i < skip1)) return;
+    col[dpos[i]] = rows[i];
+    val[dpos[i]] = diag_rest(sum[i], scale[rows[i]]);
 }
 
 // The rows of FE s in the projected iteration, a workgroup per large level: they
 // form (A_s'A_s)^-1 A_s'A_o v, so their entries are divided by d; the one on the
 // diagonal is taken out (its element of v is being written by the same launch).
-__global__ __launch_bounds__(kBlock) void k_nf_project_rows(const int32_t *__restrict__ big,
+__global__ __launch_bounds__(kBlock) void k_nf_project_rows(const int32_t *__restrict__ rows,
                                                             const double *__restrict__ sum,
-                                                            const int32_t *__restrict__ obs,
                                                             const double *__restrict__ scale,
                                                             const int32_t *__restrict__ off,
                                                             int32_t *__restrict__ col, double *__restrict__ val) {
-    const int32_t i = blockIdx.x, k = big[i], e0 = off[k], e1 = off[k + 1] - 1;
-    const double f = 1.0 / (1.0 + diag_rest(sum, i, obs, scale, k));
+    const int32_t i = blockIdx.x, k = rows[i], e0 = off[k], e1 = off[k + 1] - 1;
+    const double f = 1.0 / (1.0 + diag_rest(sum[i], scale[k]));
     for (int32_t e = e0 + threadIdx.x; e < e1; e += kBlock) val[e] *= f;
     if (threadIdx.x == 0) {
         col[e1] = col[e0];
@@ -1370,12 +1368,10 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, int64_t fa
     NRC(tmp.get(&count, 1));
     int64_t cells = 0;
     std::vector<int64_t> fe_nnz(in.G, 0);
-    m.dfe.assign(1, 0);
     for (int g = 0; g < in.G; g++) {
         fe_nnz[g] = in.nbig[g];
-        m.dfe.push_back(m.dfe.back() + in.nbig[g]);
+        m.ndiag += in.nbig[g];
     }
-    const int32_t ndiag = m.dfe.back();
     for (int x = 0; x < in.G; x++)
         for (int y = x + 1; y < in.G; y++) {
             // a: FE s where it is one of the two (the internal order keeps its levels together), else the larger
@@ -1422,7 +1418,7 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, int64_t fa
             fe_nnz[a] += nc;
             fe_nnz[b] += nc;
             m.far += (in.n[a] > kNfFarLevels ? nc : 0) + (in.n[b] > kNfFarLevels ? nc : 0);
-            if (2 * cells > nnz_max || 2 * cells + ndiag + (int64_t)kNfRow * p > INT32_MAX) {
+            if (2 * cells > nnz_max || 2 * cells + m.ndiag + (int64_t)kNfRow * p > INT32_MAX) {
                 *fits = 0;
                 return 0;
             }
@@ -1469,7 +1465,7 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, int64_t fa
             tmp.drop(list);
         }
     // rows: the entries of every pair a level takes part in, pair after pair, and a large level's diagonal
-    m.nnz = 2 * cells + ndiag;
+    m.nnz = 2 * cells + m.ndiag;
     uint32_t *cur = nullptr;
     NRC(tmp.get(&cur, p + 1));
     NRC(alloc(h, &m.off, p + 1));
@@ -1484,10 +1480,9 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, int64_t fa
         add(ps[i].offa, m.pairs[i].a);
         add(ps[i].offb, m.pairs[i].b);
     }
-    for (int g = 0; g < in.G; g++)
-        if (in.nbig[g])
-            hipLaunchKernelGGL(k_nf_add_diag, dim3(blocks_for(in.nbig[g], kBlock)), dim3(kBlock), 0, st, in.big[g],
-                               in.nbig[g], cur + in.off[g]);
+    if (m.ndiag)
+        hipLaunchKernelGGL(k_nf_add_diag, dim3(blocks_for(m.ndiag, kBlock)), dim3(kBlock), 0, st, in.big_rows,
+                           m.ndiag, cur);
     NCHK(hipGetLastError());
     NRC(solver_scan(h, cur, p, (uint32_t *)m.off));
     NCHK(hipMemcpyAsync(cur, m.off, sizeof(uint32_t) * p, hipMemcpyDeviceToDevice, st));
@@ -1507,12 +1502,12 @@ static int build(fehip_solver *h, const NfInput &in, int64_t nnz_max, int64_t fa
         add(w.offb, q.b);
         NCHK(hipGetLastError());
     }
-    NRC(alloc(h, &m.dpos, ndiag));
-    for (int g = 0; g < in.G; g++)
-        if (in.nbig[g])
-            hipLaunchKernelGGL(k_nf_place_diag, dim3(blocks_for(in.nbig[g], kBlock)), dim3(kBlock), 0, st, in.big[g],
-                               in.nbig[g], (const uint32_t *)cur + in.off[g], (int32_t)in.off[g], m.dpos + m.dfe[g], m.col);
-    NCHK(hipGetLastError());
+    if (m.ndiag) {
+        NRC(alloc(h, &m.dpos, m.ndiag));
+        hipLaunchKernelGGL(k_nf_place_diag, dim3(blocks_for(m.ndiag, kBlock)), dim3(kBlock), 0, st, in.big_rows,
+                           m.ndiag, (const uint32_t *)cur, m.dpos, m.col);
+        NCHK(hipGetLastError());
+    }
     // tiles: of the FEs before s, of s, of those after it
     // (small problems: shorter tiles, down to a wave's two loads per lane, so that
     // every CU has some)
@@ -1608,17 +1603,13 @@ int nf_values(const NfInput &in, NormalMat &m, bool projected) {
                                (const int32_t *)q.big, (const int32_t *)q.start, (const int32_t *)q.order, ca, cb,
                                (const int32_t *)q.dsta, (const int32_t *)q.dstb, m.val);
     }
-    for (int g = 0; g < in.G; g++) {
-        const int32_t n = in.nbig[g];
-        if (!n) continue;
-        if (projected && g == in.s)
-            hipLaunchKernelGGL(k_nf_project_rows, dim3((unsigned)n), dim3(kBlock), 0, in.stream, in.big[g],
-                               in.big_sum[g], in.obs[g], in.scale[g], (const int32_t *)m.off + in.off[g], m.col,
-                               m.val);
-        else
-            hipLaunchKernelGGL(k_nf_diag, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, in.stream, in.big[g], n,
-                               in.big_sum[g], in.obs[g], in.scale[g], (int32_t)in.off[g],
-                               (const int32_t *)m.dpos + m.dfe[g], m.col, m.val);
+    if (m.ndiag) {
+        const int32_t s0 = in.big0_s, ns = projected ? in.nbig[in.s] : 0;
+        hipLaunchKernelGGL(k_nf_diag, dim3(blocks_for(m.ndiag, kBlock)), dim3(kBlock), 0, in.stream, in.big_rows,
+                           m.ndiag, s0, s0 + ns, in.big_sum, in.scale, (const int32_t *)m.dpos, m.col, m.val);
+        if (ns)
+            hipLaunchKernelGGL(k_nf_project_rows, dim3((unsigned)ns), dim3(kBlock), 0, in.stream, in.big_rows + s0,
+                               in.big_sum + s0, in.scale, (const int32_t *)m.off, m.col, m.val);
     }
     m.projected = projected;
     NCHK(hipGetLastError());
