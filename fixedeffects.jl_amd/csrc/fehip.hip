@@ -290,9 +290,10 @@ static void release_spares(fehip_solver *h) {
 static void settle(fehip_solver *h) {
     if (h && !h->spares.empty() && hipStreamSynchronize(h->stream) == hipSuccess) release_spares(h);
 }
-// (declared first: it runs when a call's other locals are gone)
+// around a call (declared first: it ends when the call's other locals are gone)
 struct Settle {
     fehip_solver *h;
+    explicit Settle(fehip_solver *h) : h(h) { pool_read_limit(); }
     ~Settle() { settle(h); }
 };
 
@@ -959,6 +960,7 @@ static int create_impl(fehip_t **out, int64_t N, int32_t G, const R *const *refs
         if (nlevels[g] < 1 || nlevels[g] > (int64_t)INT32_MAX - 2)
             return fail(FEHIP_EDIM, "nlevels[" + std::to_string(g) + "] out of range");
     }
+    pool_read_limit();
     std::unique_ptr<fehip_solver> hp(new fehip_solver());
     fehip_solver *h = hp.get();
     if (const char *e = std::getenv("FEHIP_POLL_ITERS")) h->poll_iters = std::max(1, std::atoi(e));
@@ -4380,6 +4382,7 @@ int fehip_solve_residuals_panels(fehip_t *const *hs, int32_t npanels, double *co
                                  uint8_t *const *converged) {
     g_err.clear();
     if (!hs || !dY || !K || !ldY || npanels < 0) return fail(FEHIP_EARG, "bad arguments");
+    pool_read_limit();
     if (maxiter < 1) return fail(FEHIP_EARG, "maxiter must be >= 1");
     for (int32_t i = 0; i < npanels; i++) {
         if (!hs[i] || !dY[i]) return fail(FEHIP_EARG, "panel " + std::to_string(i) + ": NULL handle or column block");
@@ -4451,6 +4454,7 @@ int fehip_solve_residuals_panels_host(fehip_t *const *hs, int32_t npanels, doubl
                                       uint8_t *const *converged) {
     g_err.clear();
     if (!hs || !cols || !K || npanels < 0) return fail(FEHIP_EARG, "bad arguments");
+    pool_read_limit();
     for (int32_t i = 0; i < npanels; i++) {
         if (!hs[i] || !cols[i]) return fail(FEHIP_EARG, "panel " + std::to_string(i) + ": NULL handle or columns");
         if (K[i] < 1 || K[i] > kMaxK) return fail(FEHIP_EARG, "panel " + std::to_string(i) + ": K must be in 1..32");
@@ -4598,6 +4602,7 @@ int fehip_group(int64_t N, int32_t ncols, const int64_t *const *keys, int64_t *r
         return 0;
     }
     if (N >= (int64_t)INT32_MAX) return fail(FEHIP_EARG, "too many observations for one grouping call");
+    pool_read_limit();
     fehip_solver *h = new fehip_solver();
     hipError_t e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
     int rc = e == hipSuccess ? group_keys(h, N, ncols, keys, refs, ngroups) : fail(FEHIP_EHIP, hipGetErrorString(e));

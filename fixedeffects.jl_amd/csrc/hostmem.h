@@ -13,9 +13,7 @@ namespace fehip {
 // A block of at least `bytes` on the current device, and its real size and
 // device (for pool_put).  Its contents are undefined.  Blocks come from those
 // given back before where one of the same size class is there, else from
-// hipMalloc (after emptying the pool if that fails).  FEHIP_DEVICE_MB in the
-// environment limits what blocks may come to per device, in MB; beyond it a
-// call fails as it does where the device has no room.
+// hipMalloc (after emptying the pool if that fails).
 hipError_t pool_get(size_t bytes, void **ptr, size_t *size, int *device);
 
 // Gives a block back.  No work that uses it may be pending on any stream.
@@ -23,6 +21,11 @@ hipError_t pool_get(size_t bytes, void **ptr, size_t *size, int *device);
 void pool_put(void *ptr, size_t size, int device);
 
 constexpr size_t kPoolBytes = size_t(4) << 30;
+
+// FEHIP_DEVICE_MB in the environment limits what blocks may come to per device,
+// in MB; beyond it a call fails as it does where the device has no room.  Read
+// here, once a call of the C-ABI.
+void pool_read_limit();
 
 // Frees the blocks the pool keeps, of every device.
 void pool_trim();

@@ -73,6 +73,8 @@ struct Pool {
     }
 };
 
+std::atomic<size_t> g_limit{SIZE_MAX};  // FEHIP_DEVICE_MB, in bytes
+
 // one per device, never destroyed (handles may be closed at process exit)
 struct Pools {
     std::mutex mu;
@@ -98,8 +100,7 @@ hipError_t pool_get(size_t bytes, void **ptr, size_t *size, int *device) {
     if (e != hipSuccess) return e;
     *size = size_class(bytes);
     Pool &p = pool_of(*device);
-    const char *env = getenv("FEHIP_DEVICE_MB");
-    const size_t limit = env && *env ? (size_t)std::max(0ll, atoll(env)) << 20 : SIZE_MAX;
+    const size_t limit = g_limit.load(std::memory_order_relaxed);
     if (limit != SIZE_MAX && p.over(limit)) p.trim();
     {
         std::lock_guard<std::mutex> lk(p.mu);
@@ -128,6 +129,11 @@ void pool_put(void *ptr, size_t size, int device) {
         }
     }
     p.drop(ptr, size);
+}
+
+void pool_read_limit() {
+    const char *env = getenv("FEHIP_DEVICE_MB");
+    g_limit.store(env && *env ? (size_t)std::max(0ll, atoll(env)) << 20 : SIZE_MAX, std::memory_order_relaxed);
 }
 
 void pool_trim() {
